@@ -42,7 +42,7 @@ def _run(cmd, cwd=None):
 # Device headers embedded in the library for the lattice-specialised kernels it compiles at run
 # time (bmx_jit.cpp): their text, minus the include lines the run-time compiler resolves itself.
 JIT_HEADERS = [("bmx_jit_src_table", "bmx_table.hpp"), ("bmx_jit_src_maps", "bmx_maps.hpp"),
-               ("bmx_jit_src_tiles", "bmx_tiles.hpp")]
+               ("bmx_jit_src_fast", "bmx_fast.hpp"), ("bmx_jit_src_tiles", "bmx_tiles.hpp")]
 
 
 def write_jit_sources(path: str) -> str:

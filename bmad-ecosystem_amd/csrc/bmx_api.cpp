@@ -33,7 +33,7 @@ static int hip_fail(hipError_t e, const char *what)
 // Equal kernel arguments: the same device arrays and values (a captured launch holds them).
 static bool same_launch(const LatDesc &a, const LatDesc &b)
 {
-    return a.hdr == b.hdr && a.prm == b.prm && a.n_ele == b.n_ele && a.sp.mc2 == b.sp.mc2 &&
+    return a.hdr == b.hdr && a.prm == b.prm && a.ops == b.ops && a.n_ele == b.n_ele && a.sp.mc2 == b.sp.mc2 &&
            a.sp.p0c == b.sp.p0c && a.sp.mc2_sq == b.sp.mc2_sq && a.sp.beta0 == b.sp.beta0 &&
            a.sp.me2 == b.sp.me2 && a.sp.lez_f == b.sp.lez_f && a.sp.lez_thr == b.sp.lez_thr &&
            a.sp.rad.scale == b.sp.rad.scale && a.sp.rad.flags == b.sp.rad.flags &&
@@ -191,10 +191,8 @@ int32_t bmx_lattice_set_radiation(bmx_lattice *L, const bmx_rad_config *config)
         return set_error(BMX_ERR_ARG, "bmx_lattice_set_radiation: bad argument");
     L->host.sp.rad = rad_settings(*config);
     L->desc.sp.rad = L->host.sp.rad;
+    // runs take the descriptor by value when they are queued; those queued before keep theirs
     hipSetDevice(L->device);
-    // ordered after the context's queued work that reads the descriptor
-    HIP_TRY(hipMemcpyAsync(L->d_desc, &L->desc, sizeof(LatDesc), hipMemcpyHostToDevice, L->ctx->stream),
-            "bmx_lattice_set_radiation: copy");
     HIP_TRY(hipStreamSynchronize(L->ctx->stream), "bmx_lattice_set_radiation: sync");
     return BMX_OK;
 }
@@ -212,25 +210,39 @@ int32_t lattice_upload(bmx_ctx *ctx, HostTable &&table, bmx_lattice **out)
     L->ctx = ctx;
     L->device = ctx->device;
     hipSetDevice(ctx->device);
-    const size_t nh = L->host.hdr.size(), np = L->host.prm.size();
-    hipError_t e = hipMalloc(&L->d_hdr, nh * sizeof(EleHdr));
-    if (e == hipSuccess) e = hipMalloc(&L->d_prm, (np ? np : 1) * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&L->d_desc, sizeof(LatDesc));
-    if (e == hipSuccess) e = hipMemcpy(L->d_hdr, L->host.hdr.data(), nh * sizeof(EleHdr), hipMemcpyHostToDevice);
-    if (e == hipSuccess && np) e = hipMemcpy(L->d_prm, L->host.prm.data(), np * sizeof(double), hipMemcpyHostToDevice);
-    L->desc.hdr = L->d_hdr;
-    L->desc.prm = L->d_prm;
-    L->desc.n_ele = (int32_t)nh;
-    L->desc.rare_q = L->host.rare_q ? (L->host.rad ? 2 : 1) : 0;
-    L->desc.sp = L->host.sp;
-    if (e == hipSuccess) e = hipMemcpy(L->d_desc, &L->desc, sizeof(LatDesc), hipMemcpyHostToDevice);
+    // one device block: the table's arrays one after the other, 64-byte aligned (the operation
+    // records are read a line at a time; one spare line, since the kernels read one ahead)
+    const HostTable &t = L->host;
+    std::vector<char> img;
+    auto place = [&](const void *p, size_t bytes, size_t spare = 0) {
+        const size_t at = (img.size() + 63) / 64 * 64;
+        img.resize(at + bytes + spare);
+        if (bytes) std::memcpy(&img[at], p, bytes);
+        return at;
+    };
+    const size_t at_hdr = place(t.hdr.data(), t.hdr.size() * sizeof(EleHdr));
+    const size_t at_prm = place(t.prm.data(), t.prm.size() * sizeof(double));
+    const size_t at_fast = place(t.fast.data(), t.fast.size() * sizeof(FastEle));
+    const size_t at_blk = place(t.blk.data(), t.blk.size() * sizeof(FastBlock));
+    const size_t at_rad = place(t.rad_lines.data(), t.rad_lines.size() * sizeof(double));
+    const size_t at_ops = place(t.ops.data(), t.ops.size() * sizeof(double), kFastOpLen * sizeof(double));
+    hipError_t e = hipMalloc(&L->d_table, img.size());
+    if (e == hipSuccess) e = hipMemcpy(L->d_table, img.data(), img.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
-        hipFree(L->d_hdr);
-        hipFree(L->d_prm);
-        hipFree(L->d_desc);
+        hipFree(L->d_table);
         delete L;
         return hip_fail(e, "bmx_lattice_create: device table");
     }
+    L->desc.hdr = (const EleHdr *)(L->d_table + at_hdr);
+    L->desc.prm = (const double *)(L->d_table + at_prm);
+    L->desc.fast = (const FastEle *)(L->d_table + at_fast);
+    L->desc.blk = (const FastBlock *)(L->d_table + at_blk);
+    L->desc.rad = (const double *)(L->d_table + at_rad);
+    L->desc.ops = (const double *)(L->d_table + at_ops);
+    L->desc.n_blk = (int32_t)t.blk.size();
+    L->desc.n_ele = (int32_t)t.hdr.size();
+    L->desc.rare_q = t.rare_q ? (t.rad ? 2 : 1) : 0;
+    L->desc.sp = t.sp;
     *out = L;
     return BMX_OK;
 }
@@ -245,9 +257,8 @@ int32_t bmx_lattice_destroy(bmx_lattice *L)
     // Independent of the context's lifetime: synchronise the device, then free.
     hipSetDevice(L->device);
     hipDeviceSynchronize();
-    hipFree(L->d_hdr);
-    hipFree(L->d_prm);
-    hipFree(L->d_desc);
+    hipFree(L->d_table);
+    hipFree(L->d_cell);
     delete L;
     return BMX_OK;
 }
@@ -268,8 +279,21 @@ int32_t bmx_lattice_specialize(bmx_lattice *L)
     if (!L) return set_error(BMX_ERR_ARG, "bmx_lattice_specialize: null lattice");
     std::string err;
     const JitKernels *j = nullptr;
-    const int rc = jit_specialize(L->device, L->host, &j, err);
+    std::vector<double> stream;
+    const int rc = jit_specialize(L->device, L->host, &j, stream, err);
     if (rc != BMX_OK) return set_error(rc, "bmx_lattice_specialize: " + err);
+    if (!L->d_cell) {
+        hipSetDevice(L->device);
+        double *d = nullptr;
+        hipError_t e = hipMalloc(&d, stream.size() * sizeof(double));
+        if (e == hipSuccess) e = hipMemcpy(d, stream.data(), stream.size() * sizeof(double), hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            hipFree(d);
+            return hip_fail(e, "bmx_lattice_specialize: cell values");
+        }
+        L->d_cell = d;
+        L->desc.cell = d;
+    }
     L->jit = j;
     return BMX_OK;
 }

@@ -37,15 +37,22 @@ struct bmx_batch {
             if (L->jit != j) return nullptr;
         return j;
     }
+    // Takes up the lattices' shared cell kernels and the values each lattice got for them when it
+    // was specialised (which may be after the batch was made).
+    void take_jit()
+    {
+        cfg.jit = shared_jit();
+        if (!cfg.jit) return;
+        for (size_t i = 0; i < groups.size(); i++) groups[i].lat.cell = lats[i]->desc.cell;
+    }
     // Follow the context's map choice and the lattices' specialisation (which may be set after
     // the batch was made); a change invalidates the captured graphs.
     void refresh(bool fast)
     {
         const bool fast_changed = cfg.fast != fast;
         cfg.fast = fast;
-        const JitKernels *j = shared_jit();
-        if (!fast_changed && j == cfg.jit) return;
-        cfg.jit = j;
+        if (!fast_changed && shared_jit() == cfg.jit) return;
+        take_jit();
         if (waves_auto) cfg.waves = default_waves(cfg.fast, cfg.jit);
         if (grid_auto) cfg.grid = default_grid(device, cfg.fast, cfg.waves, cfg.jit);
         drop_graphs();
@@ -124,7 +131,7 @@ int32_t bmx_batch_create(bmx_ctx *ctx, const bmx_group *groups, int32_t n_groups
     }
     B->cfg.chunk_turns = ctx->chunk_turns;
     B->cfg.fast = ctx->fast_maps;
-    B->cfg.jit = B->shared_jit();
+    B->take_jit();
     B->waves_auto = ctx->waves == 0;
     B->cfg.waves = ctx->waves ? ctx->waves : default_waves(B->cfg.fast, B->cfg.jit);
     B->cfg.grid = default_grid(ctx->device, B->cfg.fast, B->cfg.waves, B->cfg.jit);
@@ -151,7 +158,7 @@ int32_t bmx_batch_set_run(bmx_batch *B, int32_t chunk_turns, int32_t grid, int32
     hipSetDevice(B->ctx->device);
     hipStreamSynchronize(B->ctx->stream);
     B->cfg.chunk_turns = chunk_turns;
-    B->cfg.jit = B->shared_jit();
+    B->take_jit();
     B->waves_auto = waves == 0;
     B->cfg.waves = waves ? waves : default_waves(B->cfg.fast, B->cfg.jit);
     B->grid_auto = grid <= 0;
@@ -166,10 +173,10 @@ int32_t bmx_batch_track(bmx_batch *B, int32_t n_turns, int32_t turn0)
     if (n_turns == 0 || B->groups.empty()) return BMX_OK;
     bmx_ctx *ctx = B->ctx;
     hipSetDevice(ctx->device);
-    B->refresh(ctx->fast_maps != 0);
     // the previous call's upload of the host group array must be complete before it changes
     hipError_t e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return fail(e, "bmx_batch_track");
+    B->refresh(ctx->fast_maps != 0);
     for (Group &g : B->groups) {
         g.n_turns = n_turns;
         g.turn0 = turn0;
@@ -206,13 +213,15 @@ int32_t bmx_batch_tune(bmx_batch *B, int32_t sample_turns, int32_t *chunk_out, i
     if (!B || sample_turns <= 0) return set_error(BMX_ERR_ARG, "bmx_batch_tune: bad argument");
     bmx_ctx *ctx = B->ctx;
     hipSetDevice(ctx->device);
+    hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess) return fail(e, "bmx_batch_tune");
     B->refresh(ctx->fast_maps != 0);
     const size_t n = B->n_particles;
     if (n == 0) return BMX_OK;
     // scratch SoA copy of every group's particles, restored before each candidate
     const size_t nd = n * 8, ni = n * 4;
     char *orig = nullptr, *work = nullptr;
-    hipError_t e = hipMalloc(&orig, 7 * nd + 3 * ni);
+    e = hipMalloc(&orig, 7 * nd + 3 * ni);
     if (e == hipSuccess) e = hipMalloc(&work, 7 * nd + 3 * ni);
     if (e != hipSuccess) {
         hipFree(orig);

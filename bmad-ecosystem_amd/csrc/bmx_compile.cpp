@@ -7,6 +7,7 @@
 // functions (track_a_bend.f90:139-175) and aperture geometry (check_aperture_limit.f90:358-385).
 // Anything the GPU maps do not implement is rejected with BMX_ERR_UNSUPPORTED, mirroring
 // track1_bmad's "not implemented" error (track1_bmad.f90:263-270).
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -573,6 +574,299 @@ bool finite_map(const bmx_rad_map &m)
 
 }  // namespace
 
+namespace {
+
+// The fast-path operations of one element, or false when only the general maps can take it.
+// Whatever the operations' tests leave undecided they refuse per particle (bmx_fast.hpp), so the
+// limits here only choose which elements are worth running on them:
+//  - a centred ellipse, a rectangle about the axis or no aperture at the exit; without one the
+//    test is r < 500 m, half of orbit_too_large's limit (the general maps decide beyond it);
+//  - offsets in x and y and tilts, no pitches or longitudinal offsets;
+//  - quadrupoles up to k1 L^2 = 0.7 a step (the five-term series reaches t = 1; 0.055 keeps the
+//    short series' t <= 2^-8 with room for 1 + pz down to 0.9), with dipole kicks;
+//  - bends with the simple edges: on the momentum form, strong enough that an orbit beyond
+//    orbit_too_large's 1 km fails the angle test at the exit face (g sin a >= 2.5e-4), or with a
+//    gradient up to k L^2 = 0.055.
+// The elliptical test is narrowed by 1e-12, far above its rounding: a particle it passes passes
+// the general test too.
+struct FastBuild {
+    struct Op {
+        uint32_t code;
+        double v[kFastOpLen];
+    };
+    std::vector<Op> ops;
+    bool u_open = false;      // the last operation changed px, py and left them untested
+    double x_max = 1e9, y_max = 1e9;  // bounds of |x|, |y| after the last exit test
+
+    static constexpr double kNoAperture[2] = {0, HUGE_VAL};
+
+    // rad: the element's two packed radiation maps (FO_RAD's values), or null.
+    bool element(const EleHdr &h, const double *prm, const double *rad)
+    {
+        ops.clear();
+        if (h.flags & (F_APE_ENT | F_APE_MOMENTUM)) return false;
+        if ((h.flags & F_RAD) && !rad) return false;
+        const double *ob = prm + h.off;
+        const double *ap = (h.flags & F_OFFSET) ? ob + kOffsetLen : ob;
+        const bool has_ap = h.flags & (F_APE_ENT | F_APE_EXIT | F_APE_ENT_SAME);
+        const double *q = has_ap ? ap + 4 : ap;
+        double k2 = 1, r2 = 2.5e5;
+        uint32_t rect = 0;
+        double xm = 500, ym = 500;
+        if (h.flags & F_APE_EXIT) {
+            if (h.flags & F_APE_ELLIP) {
+                if (!(h.flags & F_APE_CENTERED)) return false;
+                xm = 1 / ap[1];
+                ym = 1 / ap[3];
+                if (!(xm > 0 && ym > 0 && xm <= kMaxAp && ym <= kMaxAp)) return false;
+                k2 = (xm / ym) * (xm / ym);
+                r2 = xm * xm * (1 - 1e-12);
+            } else {
+                const double lo[2] = {ap[0], ap[2]}, hi[2] = {ap[1], ap[3]};
+                double w[2];
+                for (int k = 0; k < 2; k++) {
+                    if (lo[k] == 0 && hi[k] == 0) w[k] = 500;
+                    else if (hi[k] > 0 && lo[k] == -hi[k]) w[k] = std::fmin(hi[k], 500.0);
+                    else return false;
+                }
+                rect = FO_RECT;
+                xm = k2 = w[0];
+                ym = r2 = w[1];
+            }
+        }
+        // the aperture goes with the element's map, or, where something follows that, with a mark
+        const bool framed = h.flags & F_OFFSET;
+        const bool mark = framed || (h.flags & F_RAD);
+        auto add = [&](uint32_t code, std::initializer_list<double> v, bool last) {
+            Op o{code, {}};
+            std::copy(v.begin(), v.end(), o.v);
+            const bool test = last && !mark;
+            if (test) o.code |= rect;
+            o.v[6] = test ? k2 : kNoAperture[0];
+            o.v[7] = test ? r2 : kNoAperture[1];
+            ops.push_back(o);
+        };
+        // A momentum change before the operation's own test: bounded well below the limit, it leaves
+        // momenta beyond half the limit far outside that test; else it tests on entering.
+        auto entry = [&](bool bounded) { return u_open && !bounded ? (uint32_t)FO_UCHECK : 0u; };
+        if (h.flags & F_RAD) {
+            add(FO_RAD | entry(false), {rad[0]}, false);
+            u_open = true;
+        }
+        if (framed) {
+            // (a frame change leaves px^2 + py^2 as it is: u_open stays)
+            const double one[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
+            if (ob[2] != 0 || !std::equal(one, one + 9, ob + 4) || !std::equal(one, one + 9, ob + 13)) return false;
+            const double c = ob[22], sn = ob[23];
+            add(FO_FRAME, {c, sn, -(c * ob[0] + sn * ob[1]), -(c * ob[1] - sn * ob[0])}, false);
+        }
+        const double x_in = framed ? 1e9 : x_max, y_in = framed ? 1e9 : y_max;
+        switch (h.kind) {
+        case K_DRIFT:
+            if (q[0] != 0) {
+                add(FO_DRIFT, {q[0]}, true);
+                u_open = false;
+            } else {
+                add(FO_MARK, {}, true);
+            }
+            break;
+        case K_MARKER: add(FO_MARK, {}, true); break;
+        case K_QUAD: {
+            const double w = std::fabs(q[2]);
+            if (!(w <= 0.7)) return false;
+            add((w <= 0.055 ? FO_QUAD : FO_QUAD5) | entry(false), {q[0], q[2], q[1]}, true);
+            u_open = true;
+            break;
+        }
+        case K_QMULT: {
+            const double w = std::fabs(q[2]);
+            const int32_t edges = F_QEDGE_ENT | F_QEDGE_EXIT;
+            if (!(w <= 0.7) || h.n > 4 || (h.flags & (edges | (0xF << F_ELEC_SHIFT))) ||
+                ((h.flags >> F_ORDER_SHIFT) & 0xF) != 1)
+                return false;
+            const double kx = -q[9], ky = q[5];  // half a step's
+            const uint32_t code = w <= 0.055 ? FO_QUAD : FO_QUAD5;
+            add(FO_KICK | entry(false), {kx, ky}, false);
+            for (int32_t i = 1; i <= h.n; i++) {
+                add(code | FO_UCHECK, {q[0], q[2], q[1]}, false);
+                const double n = i == h.n ? 1 : 2;
+                add(FO_KICK, {n * kx, n * ky}, false);
+            }
+            if (!mark) add(FO_MARK, {}, true);
+            u_open = true;
+            break;
+        }
+        case K_MULT: {
+            const int32_t mask = (h.flags >> F_ORDER_SHIFT) & 0xF;
+            if (mask == 4 && (h.flags & F_MULT_NORMAL) && q[0] != 0 && h.n <= 8) {
+                const double kick = 2 * std::fabs(q[7]) * (x_in * x_in + y_in * y_in);
+                for (int32_t i = 1; i <= h.n; i++)
+                    add(FO_SEXT | (i == 1 ? entry(kick < 0.2) : (uint32_t)FO_UCHECK), {q[0], q[7], 2 * q[7]}, i == h.n);
+                u_open = true;
+            } else if (mask == 1 && (q[0] == 0 || h.n == 1)) {
+                // half kick, drift, half kick; n_step kicks at one place for a thin kicker
+                const double kx = -q[5], ky = q[1];
+                const double n = q[0] == 0 ? 2 * h.n : 1;
+                add(FO_KICK | entry(false), {n * kx, n * ky}, false);
+                if (q[0] != 0) {
+                    add(FO_DRIFT, {q[0]}, false);
+                    add(FO_KICK, {kx, ky}, false);
+                }
+                if (!mark) add(FO_MARK, {}, true);
+                u_open = true;
+            } else {
+                return false;
+            }
+            break;
+        }
+        case K_BEND: {
+            const int32_t edges = F_EDGE_ENT | F_EDGE_EXIT | F_EDGE_SIMPLE;
+            if ((h.flags & (edges | F_BEND_DRIFT)) != edges || !(h.flags & F_BEND_SERIES)) return false;
+            const double g = q[1];
+            if (!(std::fabs(g * q[5]) >= 2.5e-4)) return false;
+            add(FO_BEND | entry(2 * std::fabs(g) * y_in < 0.5), {g, q[4], q[5], q[27], q[28], q[0]}, true);
+            u_open = 2 * std::fabs(g) * ym >= 0.5;
+            break;
+        }
+        case K_BMULT: {
+            const int32_t need = F_BK1 | F_BSEMI | F_QEDGE_ENT | F_QEDGE_EXIT | F_EDGE_ENT | F_EDGE_EXIT;
+            if ((h.flags & need) != need || (h.flags & (F_MISALIGN | F_TILT | F_BEXACT)) || h.n != 1 ||
+                ((h.flags >> F_ORDER_SHIFT) & 0xF) || ((h.flags >> F_ELEC_SHIFT) & 0xF))
+                return false;
+            const double g = q[1], k1 = q[30], L = q[0], kx = k1 + g * q[2];
+            // simple edges: no edge angles, fringe integrals or edge gradients
+            for (int k : {10, 11, 13, 14, 16, 17, 19, 20})
+                if (q[k] != 0) return false;
+            if (q[2] != g || q[29] != g || q[12] != g || q[18] != g || kx == 0) return false;
+            if (!(std::fabs(kx) * L * L <= 0.055 && std::fabs(k1) * L * L <= 0.055)) return false;
+            add(FO_BEND_K1 | entry(false), {g, kx, k1, g / kx, L, L * L}, true);
+            u_open = true;
+            break;
+        }
+        default: return false;
+        }
+        if (framed) {
+            const double c = ob[22], sn = ob[23];
+            add(FO_FRAME, {c, -sn, ob[0], ob[1]}, false);
+        }
+        if (h.flags & F_RAD) {
+            add(FO_RAD | entry(false), {rad[1]}, false);
+            u_open = true;
+        }
+        if (mark) {
+            ops.push_back(Op{FO_MARK | rect, {0, 0, 0, 0, 0, 0, k2, r2}});
+        }
+        x_max = xm;
+        y_max = ym;
+        return true;
+    }
+    // after an element of the general maps, which test everything at its exit
+    void general()
+    {
+        u_open = false;
+        x_max = y_max = 1e9;
+    }
+};
+constexpr double FastBuild::kNoAperture[2];
+
+// An element's two radiation maps (block rb of its parameters) as lines for FO_RAD, and the
+// operations' packed values (bmx_fast.hpp fast_radiation). False when they do not fit the packing.
+bool pack_rad(HostTable &t, int32_t ie, const double *rb, double out[2])
+{
+    for (int e = 0; e < 2; e++) {
+        const double *m = rb + e * kRadEdge;
+        const size_t line = t.rad_lines.size() / kFastOpLen;
+        if (line >= (1u << 24) || ie + 1 >= (1 << 20)) return false;
+        uint64_t rows = 0, srows = 0, scols = 0;
+        auto put = [&](const double *v, int n, double last) {
+            double l[kFastOpLen] = {};
+            std::copy(v, v + n, l);
+            l[6] = last;
+            t.rad_lines.insert(t.rad_lines.end(), l, l + kFastOpLen);
+        };
+        put(m, 6, 0);
+        for (int i = 0; i < 6; i++) {
+            const double *r = m + 6 + 6 * i;
+            bool any = m[42 + i] != 0;
+            for (int j = 0; j < 6; j++) any |= r[j] != 0;
+            if (!any) continue;
+            rows |= 1u << i;
+            put(r, 6, m[42 + i]);
+        }
+        const double *l = m + 48;
+        for (int i = 0; i < 6; l += ++i) {
+            bool any = false;
+            for (int j = 0; j <= i; j++)
+                if (l[j] != 0) {
+                    any = true;
+                    scols |= 1u << j;
+                }
+            if (!any) continue;
+            srows |= 1u << i;
+            put(l, i + 1, 0);
+        }
+        const uint64_t at = line | (uint64_t)e << 24 | rows << 26 | srows << 32 | scols << 38 | (uint64_t)(ie + 1) << 44;
+        std::memcpy(&out[e], &at, sizeof at);
+    }
+    return true;
+}
+
+void build_fast(HostTable &t)
+{
+    const int32_t n = (int32_t)t.hdr.size();
+    t.fast.assign(n, FastEle{});
+    t.fast_open.assign(n, 0);
+    t.ops.clear();
+    t.rad_lines.clear();
+    t.blk.clear();
+    FastBuild fb;
+    FastBlock cur{};
+    auto flush = [&](int32_t e1) {
+        cur.e1 = e1;
+        if (cur.e1 > cur.e0) {
+            // a run of one operation between elements of the general maps is not worth its
+            // beginning and end: it joins them
+            if (cur.n_ops == 1) cur.n_ops = 0;
+            if (cur.n_ops == 0 && !t.blk.empty() && t.blk.back().n_ops == 0) t.blk.back().e1 = e1;
+            else t.blk.push_back(cur);
+        }
+        cur = FastBlock{};
+        cur.e0 = e1;
+        cur.op0 = (int32_t)(t.ops.size() / kFastOpLen);
+    };
+    bool general = false;  // the open block is one of the general maps
+    for (int32_t i = 0; i < n; i++) {
+        const EleHdr &h = t.hdr[i];
+        double rad[2];
+        bool has_rad = false;
+        if (h.flags & F_RAD) {
+            const int32_t q = h.off + ((h.flags & F_OFFSET) ? kOffsetLen : 0) +
+                              ((h.flags & (F_APE_ENT | F_APE_EXIT | F_APE_ENT_SAME)) ? 4 : 0) +
+                              ((h.flags & F_APE_MOMENTUM) ? 8 : 0) + kParams[h.kind];
+            has_rad = h.kind != K_THIN && pack_rad(t, i, t.prm.data() + q, rad);
+        }
+        const bool ok = fb.element(h, t.prm.data(), has_rad ? rad : nullptr) && (int)fb.ops.size() <= kFastEleOps;
+        if (!ok) fb.general();
+        if (i > cur.e0 && (ok == general || (ok && cur.n_ops + (int)fb.ops.size() > kFastBlockOps)))
+            flush(i);
+        general = !ok;
+        if (!ok) continue;
+        t.fast_open[i] = fb.u_open;
+        FastEle &fe = t.fast[i];
+        fe.op0 = (int32_t)(t.ops.size() / kFastOpLen);
+        for (const FastBuild::Op &op : fb.ops) {
+            cur.codes[cur.n_ops >> 3] |= (uint64_t)op.code << (8 * (cur.n_ops & 7));
+            cur.n_ops++;
+            fe.codes[fe.n_ops >> 3] |= (uint64_t)op.code << (8 * (fe.n_ops & 7));
+            fe.n_ops++;
+            t.ops.insert(t.ops.end(), op.v, op.v + kFastOpLen);
+        }
+    }
+    flush(n);
+}
+
+}  // namespace
+
 int compile_table(const bmx_ele *eles, int32_t n_ele, double mc2, int32_t charge, HostTable &out,
                   std::string &err, const bmx_rad_map *rad, const bmx_rad_config *rad_cfg)
 {
@@ -593,6 +887,7 @@ int compile_table(const bmx_ele *eles, int32_t n_ele, double mc2, int32_t charge
     const double e_tot = eles[0].e_tot;
     if (!(e_tot > 0)) { err = "element 1 has no reference energy"; return BMX_ERR_ARG; }
     out.sp.beta0 = p0c / e_tot;
+    out.sp.inv_beta0 = 1 / out.sp.beta0;
     {
         const double me = mc2 / e_tot;
         out.sp.me2 = me * me;
@@ -965,6 +1260,7 @@ int compile_table(const bmx_ele *eles, int32_t n_ele, double mc2, int32_t charge
         if (std::memcmp(&out.prm[ha], &out.prm[ga], 4 * sizeof(double)) != 0) continue;
         h.flags = (h.flags & ~F_APE_ENT) | F_APE_ENT_SAME;
     }
+    build_fast(out);
     return BMX_OK;
 }
 

@@ -53,6 +53,12 @@ struct HostTable {
     std::vector<double> prm;
     Species sp{};
     uint64_t kind_mask = 0;  // bit = bmx_ele key present
+    // Operations (bmx_table.hpp FastOp)
+    std::vector<FastEle> fast;       // per element; n_ops = 0: the general maps only
+    std::vector<uint8_t> fast_open;  // per element: its last operation left px, py untested
+    std::vector<double> ops;         // kFastOpLen per operation
+    std::vector<double> rad_lines;   // packed radiation maps (FO_RAD)
+    std::vector<FastBlock> blk;
     bool rare_q = false;     // some element compiled to K_QMULT or K_BMULT
     bool rad = false;        // some element carries radiation kicks (rare_q is then set too)
 };
@@ -100,7 +106,9 @@ constexpr int kTileBlock = 256;
 // Lattice-specialised tile kernels (bmx_jit.cpp): compiled at run time for a lattice that is
 // mostly one repeated cell; shared by every lattice with the same cell structure.
 struct JitKernels;
-int jit_specialize(int device, const HostTable &t, const JitKernels **out, std::string &err);
+// stream: the lattice's own operation values for these kernels (LatDesc::cell).
+int jit_specialize(int device, const HostTable &t, const JitKernels **out,
+                   std::vector<double> &stream, std::string &err);
 hipError_t jit_occupancy(const JitKernels *j, int waves, int *blocks_per_cu);
 // The cell kernels carry the stepped quadrupole (their lattice holds one).
 bool jit_rare_q(const JitKernels *j);
@@ -183,10 +191,9 @@ struct bmx_lattice {
     bmx_ctx *ctx = nullptr;
     int device = 0;
     bmx::HostTable host;
-    bmx::EleHdr *d_hdr = nullptr;
-    double *d_prm = nullptr;
+    char *d_table = nullptr;          // every device array of the table, and its descriptor
+    double *d_cell = nullptr;         // operation values of the cell kernels (specialised)
     bmx::LatDesc desc{};              // device pointers inside
-    bmx::LatDesc *d_desc = nullptr;   // one-element array for the tile kernel
     const bmx::JitKernels *jit = nullptr;  // set by bmx_lattice_specialize
 };
 

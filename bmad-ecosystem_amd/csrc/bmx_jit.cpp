@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
+#include <algorithm>
+#include <cstdint>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -24,6 +26,7 @@
 
 extern const char bmx_jit_src_table[];
 extern const char bmx_jit_src_maps[];
+extern const char bmx_jit_src_fast[];
 extern const char bmx_jit_src_tiles[];
 
 namespace bmx {
@@ -74,25 +77,216 @@ bool find_period(const HostTable &t, Period &out)
     return false;
 }
 
-std::string generate(const HostTable &t, const Period &pd, std::string &sig)
+// The operations of the element at cell position j when every cell has the same ones there
+// (their tests on entering united), else false: the general maps take it.
+bool cell_ops(const HostTable &t, const Period &pd, int32_t j, std::vector<uint32_t> &codes, bool &open)
+{
+    codes.clear();
+    open = false;
+    const int32_t n = t.fast[pd.H + j].n_ops;
+    if (n <= 0) return false;
+    codes.assign(n, 0);
+    for (int32_t c = 0; c < pd.N; c++) {
+        const int32_t i = pd.H + c * pd.P + j;
+        const FastEle &fe = t.fast[i];
+        if (fe.n_ops != n) return false;
+        open |= t.fast_open[i] != 0;
+        for (int32_t k = 0; k < n; k++) {
+            const uint32_t v = (uint32_t)(fe.codes[k >> 3] >> (8 * (k & 7)) & 255);
+            if (c > 0 && (v & ~FO_UCHECK) != (codes[k] & ~FO_UCHECK)) return false;
+            codes[k] |= v;
+        }
+    }
+    return true;
+}
+
+// Where the values of a cell's operations lie in its stream (LatDesc::cell): lines of kFastOpLen
+// doubles, an operation's values within one line (they are in scalar registers together, and
+// the next line is loaded while the operations of one run). An aperture equal to the one before
+// in every cell is kept, not stored again.
+struct CellOp {
+    int32_t j, k;        // element of the cell, operation of the element
+    uint32_t code;
+    int32_t at;          // first value in the stream
+    int32_t ap;          // its aperture's k2 in the stream (r2 next), or -1: none
+};
+struct CellPlan {
+    std::vector<CellOp> ops;
+    std::vector<char> fast, open;  // per element: on operations; the last leaves px, py untested
+    int32_t lines = 0;
+};
+
+const double *op_record(const HostTable &t, const Period &pd, int32_t c, const CellOp &o)
+{
+    return &t.ops[(size_t)kFastOpLen * (t.fast[pd.H + c * pd.P + o.j].op0 + o.k)];
+}
+
+CellPlan plan_cell(const HostTable &t, const Period &pd)
+{
+    CellPlan p;
+    p.fast.assign(pd.P, 0);
+    p.open.assign(pd.P, 0);
+    int32_t at = 0, ap = -1;
+    CellOp last{};
+    auto place = [&](int32_t n) {  // n values within one line
+        if (at % kFastOpLen + n > kFastOpLen) at += kFastOpLen - at % kFastOpLen;
+        const int32_t r = at;
+        at += n;
+        return r;
+    };
+    for (int32_t j = 0; j < pd.P; j++) {
+        std::vector<uint32_t> codes;
+        bool open;
+        if (!cell_ops(t, pd, j, codes, open)) {
+            ap = -1;
+            continue;
+        }
+        p.fast[j] = 1;
+        p.open[j] = open;
+        for (size_t k = 0; k < codes.size(); k++) {
+            CellOp o{j, (int32_t)k, codes[k], 0, -1};
+            const uint32_t kind = codes[k] & FO_KIND;
+            if (!fast_untested(kind)) {
+                bool same = ap >= 0;
+                for (int32_t c = 0; c < pd.N && same; c++) {
+                    const double *a = op_record(t, pd, c, o), *b = op_record(t, pd, c, last);
+                    same = a[6] == b[6] && a[7] == b[7];
+                }
+                if (!same) ap = place(2);
+                o.ap = ap;
+                last = o;
+            }
+            o.at = place(fast_values(kind));
+            p.ops.push_back(o);
+        }
+    }
+    p.lines = (at + kFastOpLen - 1) / kFastOpLen;
+    if (p.lines == 1) p.lines = 2;  // a line is loaded while the one before is in use
+    return p;
+}
+
+std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan, std::string &sig)
 {
     bool q_kinds = false;  // the lattice holds stepped quadrupoles or general bends
     for (const EleHdr &h : t.hdr) q_kinds |= h.kind == K_QMULT || h.kind == K_BMULT;
     std::ostringstream body, key;
     key << pd.H << ':' << pd.P << ':' << pd.N << ':' << pd.S << ':' << t.hdr.size() << ':'
         << t.hdr[pd.H].off;
+    // The cell in segments: runs of at most kFastBlockOps operations (bmx_fast.hpp), and its other
+    // elements. A segment that leaves something to the general maps (elements of theirs, or the lanes
+    // a run refused) leaves the cell loop with its element range and the next segment's
+    // number; the general maps' one call site takes the range and the loop is entered again there.
+    size_t next_op = 0;
+    // One run that is the whole cell loads the next cell's first line behind its last one and
+    // carries it over; otherwise each run loads its own first line.
+    bool carry = (int32_t)plan.ops.size() <= kFastBlockOps && !plan.ops.empty();
+    for (int32_t j = 0; j < pd.P; j++) carry = carry && plan.fast[j];
+    int32_t n_seg = 0;
+    auto leave = [&](int32_t j0, int32_t j1) {
+        std::ostringstream r;
+        r << "e0 = eb + " << j0 << "; e1 = eb + " << j1 << "; ";
+        if (j1 == pd.P) r << "seg = 0; ++c; break;";
+        else r << "seg = " << n_seg + 1 << "; break;";
+        return r.str();
+    };
+    for (int32_t j = 0; j < pd.P;) {
+        body << "            case " << n_seg << ":\n";
+        if (!plan.fast[j]) {
+            int32_t j1 = j + 1;
+            while (j1 < pd.P && !plan.fast[j1]) j1++;
+            body << "                who = ~(LaneMask)0;\n                " << leave(j, j1) << '\n';
+            n_seg++;
+            j = j1;
+            continue;
+        }
+        // elements [j, j1) in one run
+        int32_t j1 = j, n = 0;
+        size_t o1 = next_op;
+        bool open = false;
+        while (j1 < pd.P && plan.fast[j1]) {
+            size_t o = o1;
+            while (o < plan.ops.size() && plan.ops[o].j == j1) o++;
+            if (n > 0 && n + (int32_t)(o - o1) > kFastBlockOps) break;
+            n += (int32_t)(o - o1);
+            if (o > o1) open = plan.open[j1];
+            o1 = o;
+            j1++;
+        }
+        if (n > 0) {
+            // the lines the run reads
+            int32_t first_line = INT32_MAX, last_line = -1, ap = -1;
+            for (size_t k = next_op; k < o1; k++) {
+                const CellOp &o = plan.ops[k];
+                if (fast_values(o.code & FO_KIND) > 0) {
+                    first_line = std::min(first_line, o.at / kFastOpLen);
+                    last_line = std::max(last_line, o.at / kFastOpLen);
+                }
+                if (o.ap >= 0 && o.ap != ap) {
+                    ap = o.ap;
+                    first_line = std::min(first_line, o.ap / kFastOpLen);
+                    last_line = std::max(last_line, o.ap / kFastOpLen);
+                }
+            }
+            body << "            {\n"
+                 << "                FastP f = fast_get(p);\n"
+                 << "                FastE ef = en;\n"
+                 << "                LaneMask bad = 0;\n"
+                 << "                double k2 = 0, r2 = 0;\n";
+            int32_t at_line = first_line - 1;
+            if (!carry && last_line >= 0)
+                body << "                OpVec l" << first_line << " = load_op(cell + " << first_line * kFastOpLen << ");\n";
+            auto val = [&](int32_t i) {
+                return "l" + std::to_string(i / kFastOpLen) + "[" + std::to_string(i % kFastOpLen) + "]";
+            };
+            auto reach = [&](int32_t i) {  // value i's line: wait for it, then load the next
+                while (at_line < i / kFastOpLen) {
+                    at_line++;
+                    body << "                arrive(l" << at_line << ");\n";
+                    if (!carry && at_line == last_line) continue;
+                    const int32_t nx = carry ? (at_line + 1) % plan.lines : at_line + 1;
+                    body << "                " << (nx == 0 ? "" : "OpVec ") << "l" << nx << " = load_op(cell + "
+                         << (at_line + 1) * kFastOpLen << ");\n"
+                         << "                load_fence();\n";
+                }
+            };
+            ap = -1;
+            for (size_t k = next_op; k < o1; k++) {
+                const CellOp &o = plan.ops[k];
+                const int32_t nv = fast_values(o.code & FO_KIND);
+                if (o.ap >= 0 && o.ap != ap) {
+                    ap = o.ap;
+                    reach(o.ap);
+                    body << "                k2 = " << val(o.ap) << ";\n                r2 = " << val(o.ap + 1) << ";\n";
+                }
+                if (nv > 0) reach(o.at);
+                body << "                {\n                    const double v[6] = {";
+                for (int32_t i = 0; i < 6; i++) body << (i ? ", " : "") << (i < nv ? val(o.at + i) : "0.0");
+                body << "};\n                    fast_op<maps_rad(kRare)>(f, ef, " << o.code
+                     << "u, v, k2, r2, L.sp, maps_rad(kRare), ra, bad);\n                }\n";
+            }
+            if (open) body << "                fast_unstable(f, ef, bad);\n";
+            body << "                if (!bad) {\n"
+                 << "                    put(p, en, f, ef);\n"
+                 << "                } else {\n"
+                 << "                    if (!this_lane(bad)) put(p, en, f, ef);\n"
+                 << "                    who = bad;\n"
+                 << "                    " << leave(j, j1) << '\n'
+                 << "                }\n"
+                 << "            }\n";
+            n_seg++;
+        } else {
+            body << "                ;\n";
+            n_seg++;
+        }
+        next_op = o1;
+        j = j1;
+    }
     for (int32_t j = 0; j < pd.P; j++) {
         const EleHdr &h = t.hdr[pd.H + j];
-        const int32_t rel = h.off - t.hdr[pd.H].off;
-        key << '/' << h.kind << ',' << h.flags << ',' << h.n << ',' << rel;
-        // the rare set only where the element is a cavity, a quadrupole with multipoles or
-        // carries offsets or momentum windows: elsewhere pz cannot change and the exit test for
-        // rel_p < 0 drops out, as in the generic loop
-        const char *maps = (h.kind == K_RF || (h.flags & (F_OFFSET | F_APE_MOMENTUM | F_RARE_MAP))) ? "kRare" : "MAPS_NO_RF";
-        body << "            if (p.state == ST_ALIVE)\n"
-             << "                track_element<true, " << maps << ">(p, EleRef{" << h.kind << ", " << h.flags
-             << ", " << h.n << ", " << rel << "}, base, L.sp, true, e1 + " << j << ", t_abs);\n";
+        key << '/' << h.kind << ',' << h.flags << ',' << h.n << ',' << h.off - t.hdr[pd.H].off << ','
+            << (int)plan.fast[j] << (int)plan.open[j];
     }
+    for (const CellOp &o : plan.ops) key << ';' << o.j << ',' << o.code << ',' << o.at << ',' << o.ap;
     if (t.rare_q) key << "/q";
     if (t.rad) key << "/r";
     sig = key.str();
@@ -100,22 +294,73 @@ std::string generate(const HostTable &t, const Period &pd, std::string &sig)
     s << "#include <stdint.h>\n"
       << bmx_jit_src_table << '\n'
       << bmx_jit_src_maps << '\n'
+      << bmx_jit_src_fast << '\n'
       << bmx_jit_src_tiles << '\n'
       << "namespace bmx {\n"
       << "struct CellTurn {\n"
       << "    static constexpr int kRare = "
       << (t.rad ? (q_kinds ? "MAPS_RARE_QR" : "MAPS_RARE_R") : t.rare_q ? "MAPS_RARE_Q" : "MAPS_RARE") << ";\n"
+      << "    __device__ __forceinline__ static void put(Particle &p, FastE &en, const FastP &f, const FastE &ef)\n"
+      << "    {\n"
+      << "        fast_put(p, f);\n"
+      << "        if constexpr (maps_rad(kRare)) {\n"
+      << "            en = ef;\n"
+      << "            fast_put_energy(p, ef);\n"
+      << "        }\n"
+      << "    }\n"
       << "    __device__ __forceinline__ static void turn(Particle &p, const LatDesc &L, int32_t t_abs)\n"
       << "    {\n"
-      << "        const CP prm = (CP)L.prm;\n";
-    if (pd.H > 0) s << "        track_range<true, kRare>(p, L, 0, " << pd.H << ", t_abs);\n";
-    s << "        for (int32_t c = 0; c < " << pd.N << "; ++c) {\n"
+      << "        const CP cells = (CP)L.cell;\n"
+      << "        FastE en = fast_energy(p, L.sp);\n"
+      << "        const RadAt ra = {(CP)L.rad, p.id, t_abs};\n"
+      << "        bool near = !maps_rad(kRare) && near_zero<kRare>(p);\n"
+      << "        int32_t c = 0, seg = 0, e0 = 0, e1 = " << pd.H << ";\n"
+      << "        LaneMask who = ~(LaneMask)0;\n"
+      << "        bool stepwise = true, done = false;\n"
+      << "        for (;;) {\n"
       << "            c = __builtin_amdgcn_readfirstlane(c);\n"
-      << "            const CP base = prm + (" << t.hdr[pd.H].off << " + c * " << pd.S << ");\n"
-      << "            const int32_t e1 = " << pd.H + 1 << " + c * " << pd.P << ";\n"
+      << "            seg = __builtin_amdgcn_readfirstlane(seg);\n"
+      << "            e0 = __builtin_amdgcn_readfirstlane(e0);\n"
+      << "            e1 = __builtin_amdgcn_readfirstlane(e1);\n"
+      // elements [e0, e1) for the lanes of who
+      << "            if (e0 < e1) {\n"
+      << "                if (this_lane(who)) {\n"
+      << "                    track_range_fast<kRare>(p, en, L, e0, e1, t_abs, stepwise);\n"
+      << "                }\n"
+      << "                if (p.state != ST_ALIVE) break;\n"
+      << "                near = !maps_rad(kRare) && near_zero<kRare>(p);\n"
+      << "            }\n"
+      << "            if (done) break;\n"
+      // a wave with a lane near the zero orbit goes on by the tables, which have the semi-linear bend
+      << "            if (near) {\n"
+      << "                e0 = e1;\n"
+      << "                e1 = L.n_ele;\n"
+      << "                who = ~(LaneMask)0;\n"
+      << "                stepwise = false;\n"
+      << "                done = true;\n"
+      << "                continue;\n"
+      << "            }\n"
+      << "            stepwise = true;\n"
+      << "            who = 0;\n";
+    if (carry) s << "            OpVec l0 = load_op(cells + c * " << plan.lines * kFastOpLen << ");\n";
+    s << "            for (; c < " << pd.N << "; ++c) {\n"
+      << "                c = __builtin_amdgcn_readfirstlane(c);\n"
+      << "                const CP cell = cells + c * " << plan.lines * kFastOpLen << ";\n"
+      << "                const int32_t eb = " << pd.H << " + c * " << pd.P << ";\n"
+      << "                switch (seg) {\n"
       << body.str()
+      << "                default: seg = 0;\n"
+      << "                }\n"
+      << "                if (who) break;\n"
+      << "            }\n"
+      << "            if (!who) {\n"
+      << "                e0 = " << pd.H + pd.N * pd.P << ";\n"
+      << "                e1 = L.n_ele;\n"
+      << "                who = ~(LaneMask)0;\n"
+      << "                stepwise = false;\n"
+      << "                done = true;\n"
+      << "            }\n"
       << "        }\n"
-      << "        track_range<true, kRare>(p, L, " << pd.H + pd.N * pd.P << ", L.n_ele, t_abs);\n"
       << "    }\n"
       << "};\n"
       << "}  // namespace bmx\n";
@@ -138,7 +383,8 @@ std::map<std::pair<int, std::string>, std::unique_ptr<JitKernels>> g_cache;
 
 }  // namespace
 
-int jit_specialize(int device, const HostTable &t, const JitKernels **out, std::string &err)
+int jit_specialize(int device, const HostTable &t, const JitKernels **out,
+                   std::vector<double> &stream, std::string &err)
 {
     *out = nullptr;
     Period pd;
@@ -147,7 +393,20 @@ int jit_specialize(int device, const HostTable &t, const JitKernels **out, std::
         return BMX_ERR_UNSUPPORTED;
     }
     std::string sig;
-    const std::string src = generate(t, pd, sig);
+    const CellPlan plan = plan_cell(t, pd);
+    const std::string src = generate(t, pd, plan, sig);
+    // the cells' values in the plan's places, and a line that the last cell's loads may reach
+    stream.assign((size_t)kFastOpLen * ((size_t)plan.lines * pd.N + 1), 0.0);
+    for (int32_t c = 0; c < pd.N; c++)
+        for (const CellOp &o : plan.ops) {
+            double *to = &stream[(size_t)kFastOpLen * plan.lines * c];
+            const double *r = op_record(t, pd, c, o);
+            for (int i = 0; i < fast_values(o.code & FO_KIND); i++) to[o.at + i] = r[i];
+            if (o.ap >= 0) {
+                to[o.ap] = r[6];
+                to[o.ap + 1] = r[7];
+            }
+        }
     std::lock_guard<std::mutex> lock(g_mutex);
     auto &slot = g_cache[{device, sig}];
     if (slot) {
@@ -159,7 +418,7 @@ int jit_specialize(int device, const HostTable &t, const JitKernels **out, std::
         err = "hiprtcCreateProgram failed";
         return BMX_ERR_HIP;
     }
-    const char *opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=fast",
+    const char *opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=fast-honor-pragmas",
                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
     const hiprtcResult rc = hiprtcCompileProgram(prog, (int)(sizeof(opts) / sizeof(opts[0])), opts);
     if (rc != HIPRTC_SUCCESS) {

@@ -129,6 +129,19 @@ __global__ void __launch_bounds__(kBlock) k_pack_alive(
     }
 }
 
+// One element of one particle on the maps of a kernel with (Q 1, 2) or without (0) the stepped
+// elements and the radiation kicks. Returns true when it was lost at the entrance aperture.
+template <bool F, int Q>
+__device__ __forceinline__ bool track_one(Particle &p, FastE &en, const LatDesc &L, int32_t ie,
+                                          int32_t turn, bool from_prev)
+{
+    if constexpr (F)
+        return track_step<Q == 2 ? MAPS_RARE_QR : Q ? MAPS_RARE_Q : MAPS_RARE>(p, en, L, ie, turn, from_prev);
+    else
+        return track_element<F, Q == 2 ? MAPS_ALL_QR : Q ? MAPS_ALL_Q : MAPS_ALL>(
+            p, load_ele((CHdr)L.hdr + 4 * ie), (CP)L.prm, L.sp, from_prev, ie + 1, turn);
+}
+
 // One element, whole bunch: track1 (track1.f90:44-343) per live particle. Q: the kernel carries
 // the stepped quadrupole and the general bend (built for lattices that hold one).
 template <bool F, int Q>
@@ -142,9 +155,10 @@ __device__ __forceinline__ void track_element_pass(const LatDesc &L, int32_t ie,
         Particle p;
         load_particle(p, b, i);
         refresh_energy(p, L.sp);
-        if (!orbit_too_large(p))
-            track_element<F, Q == 2 ? MAPS_ALL_QR : Q ? MAPS_ALL_Q : MAPS_ALL>(p, load_ele((CHdr)L.hdr + 4 * ie), (CP)L.prm, L.sp,
-                                                      false, ie + 1, turn);
+        if (!orbit_too_large(p)) {
+            FastE en = fast_energy(p, L.sp);
+            track_one<F, Q>(p, en, L, ie, turn, false);
+        }
         store_particle(p, b, i);
         if (p.state != ST_ALIVE) {
             b.state[i] = p.state;
@@ -229,10 +243,10 @@ __global__ void __launch_bounds__(kBlock) k_track_range(LatDesc L, int32_t e0, i
             lost_e = e0 + 1;
             record_orbit(rec + i * ne * 8, p, true);
         } else {
+            FastE en = fast_energy(p, L.sp);
             for (int32_t e = e0; e <= e1; ++e) {
-                const bool at_entrance =
-                    track_element<F, Q == 2 ? MAPS_ALL_QR : Q ? MAPS_ALL_Q : MAPS_ALL>(p, load_ele((CHdr)L.hdr + 4 * e), (CP)L.prm, L.sp, e > e0, e + 1,
-                                     turn);
+                e = __builtin_amdgcn_readfirstlane(e);
+                const bool at_entrance = track_one<F, Q>(p, en, L, e, turn, e > e0);
                 passes++;
                 record_orbit(rec + (i * ne + (e - e0)) * 8, p, at_entrance);
                 if (p.state != ST_ALIVE) {

@@ -118,16 +118,37 @@ __device__ __forceinline__ double sqrt_one(double v) { return v / (sqrt(1 + v) +
 // sim_utils/special_functions/sinc.f90:15-40
 __device__ __forceinline__ double sinc(double v) { return fabs(v) < 1e-8 ? 1.0 : sin(v) / v; }
 
+// 1/v: the hardware estimate refined by two Newton steps (each squares the error), zeros,
+// infinities and NaN as the division gives them.
+__device__ __forceinline__ double recip(double v)
+{
+#pragma clang fp contract(off)
+    double y = __builtin_amdgcn_rcp(v);
+    y = fma(fma(-v, y, 1.0), y, y);
+    y = fma(fma(-v, y, 1.0), y, y);
+    return __builtin_amdgcn_div_fixup(y, v, 1.0);
+}
+
+// The functions of the energy a particle carries (Particle), from pz and bq = (beta -
+// beta0)/beta0. Written as they are to be rounded: a particle gets the same values whether it
+// kept them or is read back from memory.
+__device__ __forceinline__ void energy_functions(double pz, double bq, const Species &sp, double &rel_p,
+                                                 double &inv_rp, double &ez, double &lez)
+{
+#pragma clang fp contract(off)
+    rel_p = 1 + pz;
+    inv_rp = recip(rel_p);
+    const double pc = sp.p0c * rel_p;
+    const double a = (sp.mc2_sq * fma(pz, pz, 2 * pz)) * recip(fma(pc, pc, sp.mc2_sq));
+    ez = a * recip(sqrt(1 + a) + 1);  // sqrt_one(a)
+    const double bp = sp.beta0 * pz;
+    const double low = pz * fma(pz * pz, sp.lez_f, 1 - 1.5 * (bp * sp.beta0)) * sp.me2;
+    lez = sp.mc2 * (bp * bp) < sp.lez_thr ? low : bq;
+}
+
 __device__ __forceinline__ void refresh_energy(Particle &p, const Species &sp)
 {
-    p.rel_p = 1 + p.pz;
-    p.inv_rp = 1 / p.rel_p;
-    p.ez = sqrt_one((sp.mc2_sq * (2 * p.pz + p.pz * p.pz)) / (sqr(sp.p0c * p.rel_p) + sp.mc2_sq));
-    const double pz = p.pz;
-    if (sp.mc2 * sqr(sp.beta0 * pz) < sp.lez_thr)
-        p.lez = pz * (1 - 3 * (pz * sp.beta0 * sp.beta0) / 2 + pz * pz * sp.lez_f) * sp.me2;
-    else
-        p.lez = (p.beta - sp.beta0) / sp.beta0;
+    energy_functions(p.pz, (p.beta - sp.beta0) * sp.inv_beta0, sp, p.rel_p, p.inv_rp, p.ez, p.lez);
 }
 
 // bmad/low_level/orbit_too_large.f90:26-120 (charged particle, momentum check on).
@@ -702,7 +723,7 @@ __device__ __forceinline__ double asin_over_short(double s2)
     return fma(0.022372159090909092, s8 * s2, r);      // 63/2816
 }
 
-// sin and cos of |phi| <= 4 (an rf phase wrapped to [-pi, pi)): quadrant reduction by pi/2
+// sin and cos of |phi| <= 7 (an rf phase wrapped to [-pi, pi), a deviate's angle): quadrant reduction by pi/2
 // (two-part constant) and Taylor polynomials on |r| <= pi/4 (truncation below 1e-20).
 // Coefficients (Horner order): sin -1/19!, 1/17!, ..., -1/3!; cos 1/20!, -1/18!, ..., 1/4!.
 __constant__ const double kSinCosCoef[18] = {
@@ -712,24 +733,33 @@ __constant__ const double kSinCosCoef[18] = {
     4.110317623312165e-19, -1.5619206968586225e-16, 4.779477332387385e-14,
     -1.1470745597729725e-11, 2.08767569878681e-09, -2.755731922398589e-07,
     2.48015873015873e-05, -0.001388888888888889, 0.041666666666666664};
+template <bool LO = false>
 __device__ __forceinline__ void sincos_reduced(double phi, double *sp, double *cp)
 {
     const double kPio2Hi = 1.5707963267948966;      // pi/2 rounded to double
     const double kPio2Lo = 6.123233995736766e-17;   // pi/2 - kPio2Hi
     const double kq = rint(phi * 0.6366197723675814);  // 2/pi
-    const double r = fma(-kq, kPio2Lo, fma(-kq, kPio2Hi, phi));
+    // the reduced angle and what its rounding left (LO only): errors of half a unit in the last place
+    const double w = fma(-kq, kPio2Hi, phi);
+    const double r = fma(-kq, kPio2Lo, w);
     const double r2 = r * r;
     // sin r = r (1 - r^2/3! + ... - r^18/19!), cos r = 1 - r^2/2! + ... + r^20/20!
     CP c = launder((CP)kSinCosCoef);
     double s = c[0];
 #pragma unroll
     for (int k = 1; k < 9; k++) s = fma(s, r2, c[k]);
-    s = r * fma(s, r2, 1.0);
     double cc = c[9];
 #pragma unroll
     for (int k = 10; k < 18; k++) cc = fma(cc, r2, c[k]);
     cc = fma(cc, r2, -0.5);
-    const double co = fma(cc, r2, 1.0);
+    double co = fma(cc, r2, 1.0);
+    if constexpr (LO) {
+        const double r_lo = fma(-kq, kPio2Lo, w - r);
+        s = fma(r * r2, s, fma(r_lo, co, r));
+        co = fma(-r_lo, r, co);
+    } else {
+        s = r * fma(s, r2, 1.0);
+    }
     const int q = ((int)kq) & 3;
     *sp = q == 0 ? s : (q == 1 ? co : (q == 2 ? -s : -co));
     *cp = q == 0 ? co : (q == 1 ? -s : (q == 2 ? -co : s));
@@ -1811,23 +1841,64 @@ __device__ __forceinline__ double uniform53(uint32_t hi, uint32_t lo)
     return ((double)m + 0.5) * 0x1p-53;
 }
 
-// Six standard normal deviates for one particle at one edge of one element (ran_gauss's role in
-// track1_radiation, radiation_mod.f90:116): three Philox blocks with the counter (particle,
-// turn, element, 4 edge + block), each giving two deviates by the Box-Muller transform
-// (g = sqrt(-2 ln u1) (cos, sin)(2 pi u2)).
+// ln u for 2^-54 <= u <= 1: u = 2^e f with f in [sqrt(1/2), sqrt 2), and ln f = 2 atanh s with
+// s = (f - 1)/(f + 1), |s| <= 0.1716, by its power series (the first omitted term, s^23/23, is
+// below 4e-19 of the sum).
+__device__ __forceinline__ double log_unit(double u)
+{
+#pragma clang fp contract(off)
+    double f = __builtin_amdgcn_frexp_mant(u);  // [1/2, 1)
+    int32_t e = __builtin_amdgcn_frexp_exp(u);
+    const bool low = f < 0.7071067811865476;
+    f = low ? 2 * f : f;
+    e = low ? e - 1 : e;
+    // s to twice the precision: its rounding would be the logarithm's
+    const double n = f - 1, d = f + 1, d_lo = f - (d - 1);
+    double y = __builtin_amdgcn_rcp(d);
+    y = fma(fma(-d, y, 1.0), y, y);
+    y = fma(fma(-d, y, 1.0), y, y);
+    const double s = n * y;
+    const double s_lo = fma(-d_lo, s, fma(-d, s, n)) * y;
+    const double z = s * s;
+    double r = 0.047619047619047616;         // 1/21
+    r = fma(r, z, 0.05263157894736842);       // 1/19
+    r = fma(r, z, 0.058823529411764705);      // 1/17
+    r = fma(r, z, 0.06666666666666667);       // 1/15
+    r = fma(r, z, 0.07692307692307693);       // 1/13
+    r = fma(r, z, 0.09090909090909091);       // 1/11
+    r = fma(r, z, 0.1111111111111111);        // 1/9
+    r = fma(r, z, 0.14285714285714285);       // 1/7
+    r = fma(r, z, 0.2);                        // 1/5
+    r = fma(r, z, 0.3333333333333333);        // 1/3
+    const double s2 = 2 * s;
+    // ln 2 in two parts, the first exact in products with e
+    const double k = (double)e;
+    const double a = k * 0.6931471804855391, hi = a + s2;
+    const double lo = fma(k, 7.440617110012397e-11, fma(s2 * z, r, fma(2.0, s_lo, (a - hi) + s2)));
+    return hi + lo;
+}
+
+// A pair of standard normal deviates for one particle at one edge of one element (ran_gauss's
+// role in track1_radiation, radiation_mod.f90:116): the Philox block of the counter (particle,
+// turn, element, block) through the Box-Muller transform (g = sqrt(-2 ln u1) (cos, sin)(2 pi
+// u2)).
+__device__ __forceinline__ void gauss_pair(double &g0, double &g1, uint32_t id, int32_t turn, int32_t ix1,
+                                         int32_t block, uint32_t k0, uint32_t k1)
+{
+    const Ctr4 r = philox4x32_10(Ctr4{id, (uint32_t)turn, (uint32_t)ix1, (uint32_t)block}, k0, k1);
+    const double u1 = uniform53(r.c0, r.c1), u2 = uniform53(r.c2, r.c3);
+    const double rad = sqrt(-2 * log_unit(u1));
+    double sn, cs;
+    sincos_reduced<true>(kTwoPi * u2, &sn, &cs);
+    g0 = rad * cs;
+    g1 = rad * sn;
+}
+
+// The six deviates of one edge: blocks 4 edge + 0 .. 2.
 __device__ __forceinline__ void gauss6(double *g, uint32_t id, int32_t turn, int32_t ix1, int32_t edge,
                                     uint32_t k0, uint32_t k1)
 {
-    for (int b = 0; b < 3; b++) {
-        const Ctr4 r = philox4x32_10(Ctr4{id, (uint32_t)turn, (uint32_t)ix1, (uint32_t)(4 * edge + b)},
-                                     k0, k1);
-        const double u1 = uniform53(r.c0, r.c1), u2 = uniform53(r.c2, r.c3);
-        const double rad = sqrt(-2 * log(u1));
-        double sn, cs;
-        sincos(kTwoPi * u2, &sn, &cs);
-        g[2 * b] = rad * cs;
-        g[2 * b + 1] = rad * sn;
-    }
+    for (int b = 0; b < 3; b++) gauss_pair(g[2 * b], g[2 * b + 1], id, turn, ix1, 4 * edge + b, k0, k1);
 }
 
 // The phase-space coordinates of a particle, passed to and returned from the radiation kick

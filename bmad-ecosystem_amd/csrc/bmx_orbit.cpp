@@ -61,12 +61,15 @@ bool solve(int n, double *a, double *b)
     return true;
 }
 
-// coord_struct%beta as init_coord sets it (init_coord.f90:205-207, convert_pc_to.f90:37-41).
+// coord_struct%beta as init_coord sets it (init_coord.f90:205-207, convert_pc_to.f90:37-41), in
+// extended precision: beta then changes its last bit only where its value crosses to the next
+// double. Rounded at every step it flips from probe to probe, and each flip moves z by 1e-16 per
+// metre of bend, so the search stays in a two-cycle of that size.
 double init_beta(double pz, const Species &sp)
 {
     if (pz == 0) return sp.beta0;
-    const double pc = sp.p0c * (1 + pz);
-    return pc / std::sqrt(pc * pc + sp.mc2_sq);
+    const long double pc = (long double)sp.p0c * (1 + (long double)pz);
+    return (double)(pc / std::sqrt(pc * pc + (long double)sp.mc2 * sp.mc2));
 }
 
 // ---- normal-mode tunes (mode3_mod.f90: make_N's eigen_decomp_6mat and

@@ -151,6 +151,53 @@ constexpr int kParams[K_NKIND] = {1, 5, 9, 29, 7, 0, 32, 94, 2};
 constexpr int kRadEdge = 69;
 constexpr int kRadLen = 2 * kRadEdge;
 
+// Operations of the elements that can be tracked in runs (bmx_fast.hpp): each a record of
+// kFastOpLen doubles (64 bytes), in lattice order; an element has one or more (FastEle), or none
+// and is then always tracked by the general maps.
+//  FO_DRIFT : [0] L
+//  FO_QUAD, FO_QUAD5 : [0] L, [1] b1 L, [2] b1 (short series; five terms)
+//  FO_SEXT  : [0] step, [1] b_2 r_step/2, [2] b_2 r_step (one step)
+//  FO_BEND  : [0] g, [1] cos a, [2] sin a, [3] 1 - cos a, [4] 1/g, [5] L
+//  FO_KICK  : [0] the kick in px, [1] in py (no aperture)
+//  FO_MARK  : the aperture alone
+//  FO_BEND_K1 : [0] g, [1] k_x = k1 + g^2, [2] k1, [3] g/k_x, [4] L, [5] L^2
+//  FO_FRAME : [0] cos, [1] sin of the tilt, [2], [3] the move in x, y (no aperture)
+//  FO_RAD   : [0] the packed place of the map (fast_radiation; no aperture)
+// each with its exit aperture: [6] k2, [7] r2 (x^2 + k2 y^2 < r2; with FO_RECT
+// |x| < [6] and |y| < [7]). FO_UCHECK: px^2 + py^2 <= (1+pz)^2 is tested on entering, because the
+// operation before left it untested and this one changes the momenta before testing it.
+enum FastOp : uint32_t {
+    FO_END = 0, FO_DRIFT = 1, FO_QUAD = 2, FO_QUAD5 = 3, FO_SEXT = 4, FO_BEND = 5, FO_KICK = 6,
+    FO_MARK = 7, FO_BEND_K1 = 8, FO_FRAME = 9, FO_RAD = 10, FO_KIND = 15, FO_RECT = 16, FO_UCHECK = 32,
+};
+constexpr int kFastOpLen = 8;
+// An element's operations: records op0 .. op0 + n_ops - 1, one byte of codes each (at most
+// kFastEleOps).
+constexpr int kFastEleOps = 16;
+struct FastEle {
+    uint64_t codes[2];
+    int32_t op0, n_ops;
+};
+// The table-driven kernels track the operations in blocks of at most kFastBlockOps, one run each:
+// elements [e0, e1), whose operations start at record op0; codes holds one byte per operation.
+// n_ops = 0: elements for the general maps.
+constexpr int kFastBlockOps = 16;
+struct FastBlock {
+    uint64_t codes[2];
+    int32_t op0;
+    int32_t n_ops;
+    int32_t e0, e1;
+};
+
+// Operations without an aperture test.
+constexpr bool fast_untested(uint32_t k) { return k == FO_KICK || k == FO_FRAME || k == FO_RAD; }
+// Values of operation kind k a cell kernel reads (its record without padding and aperture).
+constexpr int fast_values(uint32_t k)
+{
+    return k == FO_DRIFT ? 1 : k == FO_QUAD || k == FO_QUAD5 || k == FO_SEXT ? 3 : k == FO_KICK ? 2
+         : k == FO_BEND || k == FO_BEND_K1 ? 6 : k == FO_FRAME ? 4 : k == FO_RAD ? 1 : 0;
+}
+
 // Radiation settings of a lattice (bmad_com%radiation_damping_on, %radiation_fluctuations_on,
 // %radiation_zero_average, %synch_rad_scale), read by the kicks of F_RAD elements.
 enum : uint32_t { RAD_DAMP = 1, RAD_FLUCT = 2, RAD_ZERO_AVERAGE = 4 };
@@ -167,6 +214,7 @@ struct Species {
     double mc2_sq;   // mc2^2
     // low_energy_z_correction.f90:22-58 constants of the (single) reference energy
     double beta0;    // p0c / E_tot
+    double inv_beta0;
     double me2;      // (mc2 / E_tot)^2
     double lez_f;    // beta0^2 (2 beta0^2 - (mc2/E_tot)^2 / 2)
     double lez_thr;  // 3e-7 E_tot
@@ -181,6 +229,13 @@ struct LatDesc {
     int32_t rare_q;  // 1 when the table holds K_QMULT or K_BMULT elements, 2 when it also has
                      // radiation kicks, else 0 (read on the host only)
     Species sp;
+    const FastEle *fast;    // the elements' operations
+    const double *ops;      // operation records (FastOp)
+    const double *rad;      // packed radiation maps (FO_RAD), in lines of kFastOpLen
+    const FastBlock *blk;   // the blocks of the lattice in order, covering every element
+    const double *cell;     // the cell kernels' operation values, in lines of kFastOpLen
+    int32_t n_blk;
+    int32_t pad;
 };
 
 // Device pointers of one beam (SoA).

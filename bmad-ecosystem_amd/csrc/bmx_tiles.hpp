@@ -4,7 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include "bmx_maps.hpp"
+#include "bmx_fast.hpp"
 
 namespace bmx {
 
@@ -118,12 +118,94 @@ __device__ __forceinline__ void track_range(Particle &p, const LatDesc &L, int32
     }
 }
 
+// Elements [e0, e1) on the operations of the lattice's blocks (bmx_fast.hpp): each block of
+// operations is one run; blocks of other elements and the lanes a run refuses go element by element (one call site, so the general maps' code is there once). For
+// live particles only. stepwise: the whole range element by element.
+template <int RARE>
+__device__ __forceinline__ void track_range_fast(Particle &p, FastE &en, const LatDesc &L, int32_t e0,
+                                                 int32_t e1, int32_t t_abs, bool stepwise = false)
+{
+    const CP ops = (CP)L.ops;
+    const FastBlock BMX_CONST *blk = (const FastBlock BMX_CONST *)L.blk;
+    int32_t b = 0;
+    if (e0 > 0 && !stepwise) {  // the block that holds e0
+        int32_t hi = L.n_blk - 1;
+        while (b < hi) {
+            b = __builtin_amdgcn_readfirstlane(b);
+            const int32_t mid = (b + hi + 1) >> 1;
+            if (blk[mid].e0 <= e0) b = mid;
+            else hi = mid - 1;
+        }
+    }
+    bool near = near_zero<RARE>(p);
+    const RadAt ra = {(CP)L.rad, p.id, t_abs};
+    for (int32_t e = e0; e < e1; ++b) {
+        b = __builtin_amdgcn_readfirstlane(b);
+        e = __builtin_amdgcn_readfirstlane(e);
+        // the block's operations [k0, n_ops) (a run may begin and end inside a block)
+        int32_t k0 = 0, n_ops = 0, end = e1;
+        if (!stepwise) {
+            end = blk[b].e1 < e1 ? blk[b].e1 : e1;
+            n_ops = blk[b].n_ops;
+            if (n_ops > 0) {
+                const FastEle BMX_CONST *fast = (const FastEle BMX_CONST *)L.fast;
+                if (end != blk[b].e1) n_ops = fast[end].op0 - blk[b].op0;
+                if (e != blk[b].e0) k0 = fast[e].op0 - blk[b].op0;
+            }
+        }
+        LaneMask redo = ~(LaneMask)0;
+        if (n_ops > 0) {
+            FastP f = fast_get(p);
+            FastE ef = en;
+            LaneMask bad = 0;
+            CP r = ops + kFastOpLen * (blk[b].op0 + k0);
+            const uint64_t w1 = blk[b].codes[1];
+            uint64_t w = k0 < 8 ? blk[b].codes[0] >> (8 * k0) : w1 >> (8 * (k0 - 8));
+            OpVec next = load_op(r);
+            for (int32_t k = k0; k < n_ops; ++k) {
+                k = __builtin_amdgcn_readfirstlane(k);
+                arrive(next);
+                const OpVec v = next;
+                r += kFastOpLen;
+                next = load_op(r);  // the table ends with a spare record
+                load_fence();
+                const uint32_t code = (uint32_t)w & 255;
+                w = k == 7 ? w1 : w >> 8;
+                fast_op<maps_rad(RARE)>(f, ef, code, v, v[6], v[7], L.sp, near, ra, bad);
+            }
+            fast_unstable(f, ef, bad);
+            redo = bad;
+            if (!this_lane(bad)) {
+                fast_put(p, f);
+                if constexpr (maps_rad(RARE)) {
+                    en = ef;
+                    fast_put_energy(p, ef);
+                }
+            }
+        }
+        if (redo) {
+            if (this_lane(redo)) {
+                for (int32_t i = e; i < end && p.state == ST_ALIVE; ++i) {
+                    i = __builtin_amdgcn_readfirstlane(i);
+                    track_step<RARE>(p, en, L, i, t_abs, true);
+                }
+            }
+            if (p.state != ST_ALIVE) break;  // a lost lane waits for the others after the loop
+            near = near_zero<RARE>(p);
+        }
+        e = end;
+    }
+}
+
 template <bool F, int RARE = MAPS_RARE>
 struct GenericTurn {
     static constexpr int kRare = RARE;
     __device__ __forceinline__ static void turn(Particle &p, const LatDesc &L, int32_t t_abs)
     {
-        track_range<F, RARE>(p, L, 0, L.n_ele, t_abs);
+        if constexpr (F) {
+            FastE en = fast_energy(p, L.sp);
+            track_range_fast<RARE>(p, en, L, 0, L.n_ele, t_abs);
+        } else track_range<F, RARE>(p, L, 0, L.n_ele, t_abs);
     }
 };
 
@@ -136,9 +218,11 @@ __device__ __forceinline__ void track_span(Particle &p, const LatDesc &L, int32_
 {
     // at most two segments (first .. end, then 0 .. rest), one call site of the element loop
     int32_t e0 = first, left = count;
-    while (left > 0) {
+    FastE en = fast_energy(p, L.sp);
+    while (left > 0 && p.state == ST_ALIVE) {
         const int32_t e1 = left < L.n_ele - e0 ? e0 + left : L.n_ele;
-        track_range<F, RARE>(p, L, e0, e1, t_abs);
+        if constexpr (F) track_range_fast<RARE>(p, en, L, e0, e1, t_abs);
+        else track_range<F, RARE>(p, L, e0, e1, t_abs);
         left -= e1 - e0;
         e0 = 0;
     }
@@ -186,9 +270,9 @@ __device__ __forceinline__ unsigned long long track_particle(Particle &p, const 
         if constexpr (SPAN) {
             if (first > 0) entrance_retest(p, L, first, turn0);
         }
-        // a wave stops once all its particles are lost
+        // a lane leaves the loop when its particle is lost, the wave when all its lanes have
         for (int32_t turn = 0; turn < n_turns; ++turn) {
-            if (!any_lane(p.state == ST_ALIVE)) break;
+            if (p.state != ST_ALIVE) break;
             if constexpr (SPAN) track_span<F, Turn::kRare>(p, L, first, count, turn0 + turn);
             else Turn::turn(p, L, turn0 + turn);
         }
