@@ -449,20 +449,15 @@ int32_t track_group(bmx_ctx *ctx, const bmx_lattice *L, bmx_beam *B, int32_t fir
     // with them
     cfg.span = first != 0 || count != L->desc.n_ele;
     const int ext = L->desc.rare_q && (cfg.span || jit_level(cfg.jit) < L->desc.rare_q) ? L->desc.rare_q : 0;
-    // Run phase (waves chosen automatically, full turns on the cell kernels): while the live
-    // particles fill more than kPhaseRounds rounds of the 4-wave kernel's resident waves, the
-    // 5-wave build (more resident waves, a few spilled registers) is faster; below that, with
-    // the beam thinned by losses, the 4-wave build is. Measured per 100-turn step of the
-    // 901-element ring: 1e6, 5.7e5 and 4.2e5 live particles (3.8, 2.2, 1.6 rounds) run 3-6%
-    // faster on 5 waves, 3.4e5 and fewer (1.3 rounds) 1-4% slower.
+    // Run phase (waves chosen automatically, full turns on the cell kernels): a beam that fills more
+    // than kPhaseRounds rounds of the 4-wave kernel's resident waves runs the 5-wave build. Both
+    // give the same bits. The rule reads the beam's size, not how many of its particles live: the
+    // count cost a kernel, a copy and a wait for the stream in each call (0.13 ms at 5e5
+    // particles, 0.35 ms at 1e6), and the builds are within 2% of each other from 1.6e5 to 1e6
+    // live particles.
     if (!ctx->waves && cfg.jit && !cfg.span && !L->host.rare_q) {
-        HIP_TRY(hipMemsetAsync(ctx->d_counter, 0, sizeof(unsigned long long), ctx->stream), "memset");
-        HIP_TRY(launch_count_alive(ctx->stream, B->d.state, B->n, ctx->d_counter), "k_count_alive");
-        unsigned long long alive = 0;
-        HIP_TRY(hipMemcpyAsync(&alive, ctx->d_counter, sizeof alive, hipMemcpyDeviceToHost, ctx->stream), "copy");
-        HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
         const double resident4 = (double)default_grid(ctx->device, true, 4, cfg.jit) * (kTileBlock / 64);
-        cfg.waves = (double)((alive + 63) / 64) >= kPhaseRounds * resident4 ? 5 : 4;
+        cfg.waves = (double)((B->n + 63) / 64) >= kPhaseRounds * resident4 ? 5 : 4;
     }
     cfg.grid = ctx->grid > 0 ? ctx->grid
                              : default_grid(ctx->device, ctx->fast_maps, cfg.waves, cfg.jit, cfg.span, ext);

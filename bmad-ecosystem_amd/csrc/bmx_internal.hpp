@@ -145,7 +145,7 @@ hipError_t enqueue_run(hipStream_t s, RunBuffers &rb, const Group *h_groups, int
 // without spilling; generic fast maps 5; reference maps 3, whose 4- and 5-wave builds spill).
 // Cell kernels that carry the stepped quadrupole or the general bend are all built for 2 waves per
 // SIMD (their longer maps would spill otherwise), whichever variant is asked for.
-// The live-particle rounds of the 4-wave cell kernel above which the 5-wave build runs.
+// The rounds of the 4-wave cell kernel's resident waves above which a beam runs the 5-wave build.
 constexpr double kPhaseRounds = 1.45;
 inline int32_t default_waves(bool fast, const JitKernels *jit = nullptr)
 {
