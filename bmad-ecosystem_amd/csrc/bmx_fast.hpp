@@ -479,17 +479,48 @@ __device__ __forceinline__ void arrive(const OpVec &v)
     load_fence();
 }
 
+// What the next element by track_step starts from, read while the one before it is tracked: the
+// element's operation codes and its first operation record. The records of a lattice follow one
+// another in the order of its elements.
+struct StepAhead {
+    uint64_t codes[2];
+    int32_t n_ops;
+    CP r;       // the record in op
+    OpVec op;
+};
+
+__device__ __forceinline__ void step_codes(StepAhead &s, const FastEle BMX_CONST *fe)
+{
+    s.codes[0] = fe->codes[0];
+    s.codes[1] = fe->codes[1];
+    s.n_ops = fe->n_ops;
+}
+
+__device__ __forceinline__ StepAhead step_at(const LatDesc &L, int32_t e)
+{
+    const FastEle BMX_CONST *fe = (const FastEle BMX_CONST *)L.fast + e;
+    StepAhead s;
+    step_codes(s, fe);
+    s.r = (CP)L.ops + kFastOpLen * fe->op0;
+    s.op = load_op(s.r);
+    return s;
+}
+
 // One element for the active (live) lanes, by its definition: its operations where their tests
 // hold, else the general map. RARE: the map set of elements on the rare path (bmx_maps.hpp).
-// from_prev as track_element; e is wave-uniform. Returns true when the particle was lost at the
-// entrance aperture.
-template <int RARE>
+// from_prev as track_element; e is wave-uniform. AHEAD: s is step_at(L, e) and becomes that of
+// element e + 1 (of the last one again at the end of the lattice): a wave that goes through the
+// elements one by one spends its time waiting for these tables, one read after the other, unless
+// they are read ahead. Returns true when the particle was lost at the entrance aperture.
+template <int RARE, bool AHEAD>
 __device__ __forceinline__ bool track_step(Particle &p, FastE &en, const LatDesc &L, int32_t e,
-                                           int32_t t_abs, bool from_prev)
+                                           int32_t t_abs, bool from_prev, StepAhead &s)
 {
     const CHdr h = (CHdr)L.hdr + 4 * e;
-    const FastEle BMX_CONST *fe = (const FastEle BMX_CONST *)L.fast + e;
-    const int32_t n_ops = fe->n_ops;
+    const int32_t after = e + 1 < L.n_ele ? e + 1 : e;
+    const FastEle BMX_CONST *fe = (const FastEle BMX_CONST *)L.fast + after;
+    if constexpr (!AHEAD) step_codes(s, (const FastEle BMX_CONST *)L.fast + e);
+    const int32_t n_ops = s.n_ops;
     LaneMask redo = ~(LaneMask)0;
     if (n_ops > 0) {
         const bool near = near_zero<RARE>(p);
@@ -501,14 +532,26 @@ __device__ __forceinline__ bool track_step(Particle &p, FastE &en, const LatDesc
         if (!from_prev && (h[1] & F_APE_ENT_SAME))
             bad = lanes(aperture_fails(p, h[1] & ~F_APE_CENTERED,
                                        (CP)L.prm + h[3] + ((h[1] & F_OFFSET) ? kOffsetLen : 0)));
-        CP r = (CP)L.ops + kFastOpLen * fe->op0;
-        uint64_t w = fe->codes[0];
+        uint64_t w = s.codes[0];
+        const uint64_t w1 = s.codes[1];
+        if constexpr (!AHEAD) s.r = (CP)L.ops + kFastOpLen * ((const FastEle BMX_CONST *)L.fast + e)->op0;
         for (int32_t k = 0; k < n_ops; ++k) {
             k = __builtin_amdgcn_readfirstlane(k);
-            const OpVec v = load_op(r);
-            fast_op<maps_rad(RARE)>(f, ef, (uint32_t)w & 255, v, v[6], v[7], L.sp, near, ra, bad);
-            r += kFastOpLen;
-            w = k == 7 ? fe->codes[1] : w >> 8;
+            OpVec v;
+            if constexpr (AHEAD) {
+                arrive(s.op);
+                v = s.op;
+                s.r += kFastOpLen;
+                s.op = load_op(s.r);  // the table ends with a spare record
+                if (k == 0) step_codes(s, fe);
+                load_fence();
+            } else {
+                v = load_op(s.r);
+                s.r += kFastOpLen;
+            }
+            const uint32_t code = (uint32_t)w & 255;
+            w = k == 7 ? w1 : w >> 8;
+            fast_op<maps_rad(RARE)>(f, ef, code, v, v[6], v[7], L.sp, near, ra, bad);
         }
         fast_unstable(f, ef, bad);
         if (!this_lane(bad)) {
@@ -530,6 +573,7 @@ __device__ __forceinline__ bool track_step(Particle &p, FastE &en, const LatDesc
                 entrance = track_element<true, MAPS_NO_RF>(p, load_ele(h), (CP)L.prm, L.sp, from_prev, e + 1, t_abs);
             }
         }
+        if constexpr (AHEAD) s = step_at(L, after);  // read again, not held through the general maps
     }
     return entrance;
 }

@@ -133,33 +133,57 @@ __global__ void __launch_bounds__(kBlock) k_pack_alive(
 // elements and the radiation kicks. Returns true when it was lost at the entrance aperture.
 template <bool F, int Q>
 __device__ __forceinline__ bool track_one(Particle &p, FastE &en, const LatDesc &L, int32_t ie,
-                                          int32_t turn, bool from_prev)
+                                          int32_t turn, bool from_prev, StepAhead &s)
 {
     if constexpr (F)
-        return track_step<Q == 2 ? MAPS_RARE_QR : Q ? MAPS_RARE_Q : MAPS_RARE>(p, en, L, ie, turn, from_prev);
+        return track_step<Q == 2 ? MAPS_RARE_QR : Q ? MAPS_RARE_Q : MAPS_RARE, true>(p, en, L, ie, turn, from_prev, s);
     else
         return track_element<F, Q == 2 ? MAPS_ALL_QR : Q ? MAPS_ALL_Q : MAPS_ALL>(
             p, load_ele((CHdr)L.hdr + 4 * ie), (CP)L.prm, L.sp, from_prev, ie + 1, turn);
 }
 
+// A coordinate goes back to memory where some particle of the wave changed it (compared as bits),
+// and then for all of them, so that lines are written whole.
+__device__ __forceinline__ void store_changed(double v, double was, double *__restrict__ d, int64_t i)
+{
+    if (lanes(__double_as_longlong(v) != __double_as_longlong(was))) d[i] = v;
+}
+
 // One element, whole bunch: track1 (track1.f90:44-343) per live particle. Q: the kernel carries
 // the stepped quadrupole and the general bend (built for lattices that hold one).
+//
+// Bound by memory: the state and seven coordinates come in with one wait (a dead particle's
+// coordinates are read as well: waiting for its state first would double the latency), and only
+// what the element changed goes out (a drift 3 of the 7 arrays, a magnet 5).
 template <bool F, int Q>
 __device__ __forceinline__ void track_element_pass(const LatDesc &L, int32_t ie, int32_t turn,
                                                    const BeamPtrs &b, int64_t n,
                                                    unsigned long long *work)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const bool active = i < n && b.state[i] == ST_ALIVE;
-    if (active) {
-        Particle p;
+    StepAhead s = F ? step_at(L, ie) : StepAhead{};
+    Particle p;
+    int32_t state = 0;
+    if (i < n) {
+        state = b.state[i];
         load_particle(p, b, i);
+    }
+    const bool active = state == ST_ALIVE;
+    const LaneMask live = lanes(active);
+    if (active) {
+        const Particle was = p;
         refresh_energy(p, L.sp);
         if (!orbit_too_large(p)) {
             FastE en = fast_energy(p, L.sp);
-            track_one<F, Q>(p, en, L, ie, turn, false);
+            track_one<F, Q>(p, en, L, ie, turn, false, s);
         }
-        store_particle(p, b, i);
+        store_changed(p.x, was.x, b.x, i);
+        store_changed(p.px, was.px, b.px, i);
+        store_changed(p.y, was.y, b.y, i);
+        store_changed(p.py, was.py, b.py, i);
+        store_changed(p.z, was.z, b.z, i);
+        store_changed(p.pz, was.pz, b.pz, i);
+        store_changed(p.beta, was.beta, b.beta, i);
         if (p.state != ST_ALIVE) {
             b.state[i] = p.state;
             b.loss_ele[i] = ie + 1;
@@ -168,15 +192,11 @@ __device__ __forceinline__ void track_element_pass(const LatDesc &L, int32_t ie,
     }
     // one atomic per workgroup: the waves' counts summed in LDS
     if (!work) return;
-    unsigned long long s = active ? 1ull : 0ull;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    __shared__ unsigned long long part[kBlock / 64];
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    __shared__ uint32_t part[kBlock / 64];
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = (uint32_t)__popcll(live);
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned long long t = 0;
-        for (int w = 0; w < kBlock / 64; w++) t += part[w];
+        unsigned long long t = 0;        for (int w = 0; w < kBlock / 64; w++) t += part[w];
         if (t) atomicAdd(work + blockIdx.x % kWorkSlots, t);
     }
 }
@@ -224,13 +244,16 @@ __device__ __forceinline__ void record_orbit(double *r, const Particle &p, bool 
     r[7] = (double)p.state;
 }
 
+// One wave per workgroup: a record is 64 bytes of its particle's own row, so a wave's store meets
+// 64 lines, and few waves (a handful of particles through a ring) want a compute unit each.
+constexpr int kRecordBlock = 64;
 template <bool F, int Q>
-__global__ void __launch_bounds__(kBlock) k_track_range(LatDesc L, int32_t e0, int32_t e1,
+__global__ void __launch_bounds__(kRecordBlock) k_track_range(LatDesc L, int32_t e0, int32_t e1,
                                                         int32_t turn, BeamPtrs b, int64_t n,
                                                         double *__restrict__ rec,
                                                         unsigned long long *work)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * kRecordBlock + threadIdx.x;
     const bool active = i < n && b.state[i] == ST_ALIVE;
     unsigned long long passes = 0;
     if (active) {
@@ -244,9 +267,10 @@ __global__ void __launch_bounds__(kBlock) k_track_range(LatDesc L, int32_t e0, i
             record_orbit(rec + i * ne * 8, p, true);
         } else {
             FastE en = fast_energy(p, L.sp);
+            StepAhead s = F ? step_at(L, e0) : StepAhead{};
             for (int32_t e = e0; e <= e1; ++e) {
                 e = __builtin_amdgcn_readfirstlane(e);
-                const bool at_entrance = track_one<F, Q>(p, en, L, e, turn, e > e0);
+                const bool at_entrance = track_one<F, Q>(p, en, L, e, turn, e > e0, s);
                 passes++;
                 record_orbit(rec + (i * ne + (e - e0)) * 8, p, at_entrance);
                 if (p.state != ST_ALIVE) {
@@ -430,10 +454,10 @@ hipError_t launch_track_range(hipStream_t s, const LatDesc &lat, int32_t e0, int
                               int32_t turn, const BeamPtrs &b, int64_t n, double *d_rec,
                               unsigned long long *d_work, bool fast)
 {
-    int64_t grid = (n + kBlock - 1) / kBlock;
+    int64_t grid = (n + kRecordBlock - 1) / kRecordBlock;
     if (grid <= 0) return hipSuccess;
 #define BMX_RANGE(F, Q) \
-    hipLaunchKernelGGL((k_track_range<F, Q>), dim3((unsigned)grid), dim3(kBlock), 0, s, lat, e0, e1, turn, b, n, d_rec, d_work)
+    hipLaunchKernelGGL((k_track_range<F, Q>), dim3((unsigned)grid), dim3(kRecordBlock), 0, s, lat, e0, e1, turn, b, n, d_rec, d_work)
     if (lat.rare_q == 2) {
         if (fast) BMX_RANGE(true, 2);
         else BMX_RANGE(false, 2);

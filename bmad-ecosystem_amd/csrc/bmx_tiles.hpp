@@ -119,8 +119,11 @@ __device__ __forceinline__ void track_range(Particle &p, const LatDesc &L, int32
 }
 
 // Elements [e0, e1) on the operations of the lattice's blocks (bmx_fast.hpp): each block of
-// operations is one run; blocks of other elements and the lanes a run refuses go element by element (one call site, so the general maps' code is there once). For
-// live particles only. stepwise: the whole range element by element.
+// operations is one run; blocks of other elements and the lanes a run refuses go element by
+// element (one call site, so the general maps' code is there once). For live particles only.
+// stepwise: the whole range element by element. Neither the next block nor the next element is
+// read ahead here: the registers that takes are those of the general maps, and long beams lost
+// 5% (generic kernel, 150001 particles, 10 turns: 4.51 -> 4.78 ms), few particles gained nothing.
 template <int RARE>
 __device__ __forceinline__ void track_range_fast(Particle &p, FastE &en, const LatDesc &L, int32_t e0,
                                                  int32_t e1, int32_t t_abs, bool stepwise = false)
@@ -187,7 +190,8 @@ __device__ __forceinline__ void track_range_fast(Particle &p, FastE &en, const L
             if (this_lane(redo)) {
                 for (int32_t i = e; i < end && p.state == ST_ALIVE; ++i) {
                     i = __builtin_amdgcn_readfirstlane(i);
-                    track_step<RARE>(p, en, L, i, t_abs, true);
+                    StepAhead s;
+                    track_step<RARE, false>(p, en, L, i, t_abs, true, s);
                 }
             }
             if (p.state != ST_ALIVE) break;  // a lost lane waits for the others after the loop
