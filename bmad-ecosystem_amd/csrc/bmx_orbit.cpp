@@ -15,6 +15,7 @@
 // zero, as closed_orbit_calc turns them off); n_dim = 6 closes all six with the rf on.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstring>
@@ -245,25 +246,25 @@ int32_t bmx_closed_orbit(bmx_ctx *ctx, bmx_lattice *const *lats, int32_t n_lat, 
     // fluctuations off, and damping too for n_dim = 4 (closed_orbit_calc.f90:264, 322)
     Lattices held;
     std::vector<bmx_lattice *> use(lats, lats + n_lat);
+    const uint32_t rad_off = n_dim == 4 ? RAD_FLUCT | RAD_DAMP : RAD_FLUCT;
     for (int32_t i = 0; i < n_lat; i++) {
-        HostTable t = lats[i]->host;
-        bool changed = false;
-        const uint32_t rad_keep = n_dim == 4 ? ~(RAD_FLUCT | RAD_DAMP) : ~RAD_FLUCT;
-        if (t.sp.rad.flags & ~rad_keep) {
-            t.sp.rad.flags &= rad_keep;
-            changed = true;
-        }
-        if (n_dim == 4) {
+        // the lattice itself where there is nothing to switch off: a table is copied only to be
+        // changed (the copies of 256 rings of 901 elements are 2/3 of a six-dimensional search)
+        const HostTable &own = lats[i]->host;
+        const auto is_rf = [](const EleHdr &h) { return h.kind == K_RF; };
+        const bool rf = n_dim == 4 && std::any_of(own.hdr.begin(), own.hdr.end(), is_rf);
+        if (!rf && !(own.sp.rad.flags & rad_off)) continue;
+        HostTable t = own;
+        t.sp.rad.flags &= ~rad_off;
+        if (rf) {
             for (const EleHdr &h : t.hdr)
-                if (h.kind == K_RF) {
+                if (is_rf(h)) {
                     const int32_t q = h.off + ((h.flags & F_OFFSET) ? kOffsetLen : 0) +
                                       ((h.flags & (F_APE_ENT | F_APE_EXIT | F_APE_ENT_SAME)) ? 4 : 0) +
                                       ((h.flags & F_APE_MOMENTUM) ? 8 : 0);
                     t.prm[q + 1] = 0;  // voltage
-                    changed = true;
                 }
         }
-        if (!changed) continue;
         bmx_lattice *L = nullptr;
         const int32_t rc = lattice_upload(ctx, std::move(t), &L);
         if (rc != BMX_OK) return rc;
