@@ -407,6 +407,22 @@ int32_t bmx_beam_count_alive(bmx_beam *B, int64_t *n_alive)
 
 namespace bmx {
 
+// A tracking launch, between an event pair when the context times its kernels.
+template <class Launch> static hipError_t launch_timed(bmx_ctx *ctx, Launch launch)
+{
+    if (!ctx->profile) return launch();
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipError_t e = ctx->timer.take(&ev0);
+    if (e == hipSuccess) e = ctx->timer.take(&ev1);
+    if (e == hipSuccess) e = hipEventRecord(ev0, ctx->stream);
+    if (e == hipSuccess) e = launch();
+    if (e == hipSuccess) {
+        e = hipEventRecord(ev1, ctx->stream);
+        ctx->timer.pending.emplace_back(ev0, ev1);
+    }
+    return e;
+}
+
 // Persistent tracking of one group: n_turns turns of `count` elements from element `first`
 // (0-based), turn indices turn0 ... (bmx_table.hpp Group). fixed: run buffers of a fixed size
 // to use instead of the context's (which grow by allocation); the caller has checked that the
@@ -422,23 +438,6 @@ int32_t track_group(bmx_ctx *ctx, const bmx_lattice *L, bmx_beam *B, int32_t fir
     if (B->n >= (int64_t)UINT32_MAX) return set_error(BMX_ERR_ARG, w + ": more than 2^32-1 particles");
     if (n_turns == 0 || B->n == 0 || count == 0) return BMX_OK;
     hipSetDevice(ctx->device);
-    // the previous call's group upload must have been consumed before the host copy changes
-    HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-    RunBuffers *rb = fixed;
-    if (!rb) {
-        rb = &ctx->run;
-        rb->device = ctx->device;
-        HIP_TRY(rb->reserve(1, (size_t)B->n, (size_t)(B->n + 63) / 64), "run buffers");
-    }
-    Group &g = ctx->group;
-    g.lat = L->desc;
-    g.b = B->d;
-    g.n = (uint32_t)B->n;
-    g.list_off = 0;
-    g.n_turns = n_turns;
-    g.turn0 = turn0;
-    g.first = first;
-    g.count = count;
     RunConfig cfg;
     cfg.chunk_turns = ctx->chunk_turns;
     cfg.fast = ctx->fast_maps;
@@ -463,7 +462,32 @@ int32_t track_group(bmx_ctx *ctx, const bmx_lattice *L, bmx_beam *B, int32_t fir
                              : default_grid(ctx->device, ctx->fast_maps, cfg.waves, cfg.jit, cfg.span, ext);
     cfg.timer = ctx->profile ? &ctx->timer : nullptr;
     ctx->last = {cfg.chunk_turns, cfg.grid, cfg.waves};
-    HIP_TRY(enqueue_run(ctx->stream, *rb, &g, 1, true, n_turns, cfg, ctx->d_work), "k_track_tiles");
+    Group g{};
+    g.lat = L->desc;
+    g.b = B->d;
+    g.n = (uint32_t)B->n;
+    g.n_turns = n_turns;
+    g.turn0 = turn0;
+    g.first = first;
+    g.count = count;
+    // a span of one chunk whose waves fit on the card together: one launch (k_track_direct)
+    if (cfg.span && (cfg.chunk_turns <= 0 || n_turns <= cfg.chunk_turns) &&
+        (B->n + 63) / 64 <= (int64_t)cfg.grid * (kTileBlock / 64)) {
+        HIP_TRY(launch_timed(ctx, [&] {
+                    return launch_track_direct(ctx->stream, g, ctx->d_work, cfg.fast, L->desc.rare_q);
+                }), "k_track_direct");
+        return BMX_OK;
+    }
+    // the previous call's group upload must have been consumed before the host copy changes
+    HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    RunBuffers *rb = fixed;
+    if (!rb) {
+        rb = &ctx->run;
+        rb->device = ctx->device;
+        HIP_TRY(rb->reserve(1, (size_t)B->n, (size_t)(B->n + 63) / 64), "run buffers");
+    }
+    ctx->group = g;
+    HIP_TRY(enqueue_run(ctx->stream, *rb, &ctx->group, 1, true, n_turns, cfg, ctx->d_work), "k_track_tiles");
     return BMX_OK;
 }
 

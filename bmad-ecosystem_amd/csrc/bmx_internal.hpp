@@ -44,6 +44,8 @@ hipError_t launch_step_turn(hipStream_t s, int32_t *d_turn, bool set, int32_t v)
 hipError_t launch_track_range(hipStream_t s, const LatDesc &lat, int32_t e0, int32_t e1,
                               int32_t turn, const BeamPtrs &b, int64_t n, double *d_rec,
                               unsigned long long *d_work, bool fast);
+// One group's run as one launch on its beam's arrays (k_track_direct).
+hipError_t launch_track_direct(hipStream_t s, const Group &g, unsigned long long *d_work, bool fast, int ext);
 hipError_t launch_count_alive(hipStream_t s, const int32_t *state, int64_t n,
                               unsigned long long *d_out);
 

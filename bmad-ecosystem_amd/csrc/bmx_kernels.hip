@@ -32,6 +32,32 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(W))
                                                cnt_out, tile_ctr, chunk_off, chunk_turns, work);
 }
 
+// A run of one group that is a single chunk, straight from its beam's arrays and back, one wave per
+// workgroup: a span of elements for a beam whose waves all fit on the card at once. The tile
+// kernels' way there is a copy and four launches, of which only the last tracks: 50 of 109 us for
+// 100 elements and 5003 particles. A beam of more waves than fit goes that way, since packing the
+// live particles first takes the dead lanes out of its waves.
+constexpr int kDirectBlock = 64;
+template <bool F, int W, int RARE>
+__global__ void __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(W))) k_track_direct(
+    Group G, unsigned long long *work)
+{
+    const uint32_t i = blockIdx.x * kDirectBlock + threadIdx.x;
+    unsigned long long passes = 0;
+    Particle p;
+    int32_t state = 0;
+    if (i < G.n) {
+        state = G.b.state[i];
+        load_particle(p, G.b, i);
+    }
+    if (state == ST_ALIVE) {
+        passes = track_particle<F, GenericTurn<F, RARE>, true>(p, G.lat, G.n_turns, G.turn0, G.first, G.count);
+        if (p.state != ST_ALIVE) store_lost(p, G.b, i);
+        else store_particle(p, G.b, i);
+    }
+    add_work(work, passes);
+}
+
 // Builds the wave tiles of the next chunk from the alive counts per group (cnt_in; nullptr
 // for the first chunk: every particle of each group, indexed directly) and resets the counters
 // the next chunk appends to. One workgroup of kBuildThreads threads: a scan of the per-group
@@ -374,6 +400,21 @@ hipError_t launch_pack_alive(hipStream_t s, int grid, const Group *d_groups,
     if (grid <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_pack_alive, dim3((unsigned)grid), dim3(kBlock), 0, s, d_groups, d_tiles,
                        d_n_tiles, d_pk_out, stride, d_cnt_out);
+    return hipGetLastError();
+}
+
+hipError_t launch_track_direct(hipStream_t s, const Group &g, unsigned long long *d_work, bool fast, int ext)
+{
+    const dim3 grid((g.n + kDirectBlock - 1) / kDirectBlock), block(kDirectBlock);
+#define BMX_DIRECT(W, RARE)                                                                     \
+    do {                                                                                        \
+        if (fast) hipLaunchKernelGGL((k_track_direct<true, W, RARE>), grid, block, 0, s, g, d_work); \
+        else hipLaunchKernelGGL((k_track_direct<false, W, RARE>), grid, block, 0, s, g, d_work);     \
+    } while (0)
+    if (ext == 2) BMX_DIRECT(kExtWaves, MAPS_RARE_QR);
+    else if (ext) BMX_DIRECT(kExtWaves, MAPS_RARE_Q);
+    else BMX_DIRECT(kSpanWaves, MAPS_RARE);
+#undef BMX_DIRECT
     return hipGetLastError();
 }
 
