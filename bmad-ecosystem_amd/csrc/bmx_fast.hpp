@@ -354,6 +354,38 @@ struct RadAt {
     int32_t turn;
 };
 
+// The deviates of the columns `cols` of stoc_mat, in pairs (at: see fast_radiation).
+__device__ __forceinline__ void rad_deviates(double *g, uint64_t at, uint32_t cols, const Species &sp,
+                                             const RadAt &ra)
+{
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+    const int32_t edge = lo >> 24 & 1, ix1 = (int32_t)(hi >> 12);
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        g[2 * b] = g[2 * b + 1] = 0;
+        if (cols >> (2 * b) & 3)
+            gauss_pair(g[2 * b], g[2 * b + 1], ra.id, ra.turn, ix1, 4 * edge + b, sp.rad.key0, sp.rad.key1);
+    }
+}
+
+// The kicked coordinates back in place; energy: pz may have changed.
+__device__ __forceinline__ void rad_leave(FastP &f, FastE &en, const double *v, bool energy, const Species &sp,
+                                          LaneMask &bad)
+{
+    f.x = v[0];
+    f.px = v[1];
+    f.y = v[2];
+    f.py = v[3];
+    f.z = v[4];
+    bad |= lanes(!(v[5] > -0.5));
+    if (energy) {
+        en.pz = v[5];
+        energy_functions(en.pz, en.bq, sp, en.rel_p, en.inv_rp, en.ez, en.lez);
+        en.ir2 = en.inv_rp * en.inv_rp;
+    }
+}
+
 // track1_radiation (radiation_mod.f90:61-147) at one end of an element, as rad_kick, on a map with
 // its zero parts left out: `at` packs the map's first line in the lattice's radiation lines (low
 // 24 bits), the edge (bit 24), the rows of damp_dmat and xfer_damp_vec that are not zero (bits 26-31), the
@@ -361,7 +393,8 @@ struct RadAt {
 // bit 44). Lines of kFastOpLen values: ref_orb; then for each damping row its six coefficients and
 // xfer_damp_vec; then for each stochastic row its coefficients. A row or column of zeros adds
 // nothing to finite coordinates (others fail the tests), and a pair of deviates whose two columns
-// are zero is not drawn: each pair comes from a counter of its own.
+// are zero is not drawn: each pair comes from a counter of its own. The cell kernels have this
+// written out instead, for the coefficients that are not zero in some cell (bmx_jit.cpp).
 __device__ __forceinline__ void fast_radiation(FastP &f, FastE &en, uint64_t at, const Species &sp,
                                                const RadAt &ra, LaneMask &bad)
 {
@@ -369,7 +402,6 @@ __device__ __forceinline__ void fast_radiation(FastP &f, FastE &en, uint64_t at,
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
     CP m = ra.maps + (size_t)kFastOpLen * (lo & 0xFFFFFF);
-    const int32_t edge = lo >> 24 & 1, ix1 = (int32_t)(hi >> 12);
     const uint32_t rows = lo >> 26, srows = hi & 63, scols = hi >> 6 & 63;
     double v[6] = {f.x, f.px, f.y, f.py, f.z, en.pz};
     bad |= lanes(!(fabs(f.z) < 1e30));
@@ -395,12 +427,7 @@ __device__ __forceinline__ void fast_radiation(FastP &f, FastE &en, uint64_t at,
     }
     if (sp.rad.flags & RAD_FLUCT) {
         double g[6];
-#pragma unroll
-        for (int b = 0; b < 3; b++) {
-            g[2 * b] = g[2 * b + 1] = 0;
-            if (scols >> (2 * b) & 3)
-                gauss_pair(g[2 * b], g[2 * b + 1], ra.id, ra.turn, ix1, 4 * edge + b, sp.rad.key0, sp.rad.key1);
-        }
+        rad_deviates(g, at, scols, sp, ra);
         CP r = m + kFastOpLen * (1 + __builtin_popcount(rows));
 #pragma unroll
         for (int i = 0; i < 6; i++) {
@@ -414,17 +441,7 @@ __device__ __forceinline__ void fast_radiation(FastP &f, FastE &en, uint64_t at,
             }
         }
     }
-    f.x = v[0];
-    f.px = v[1];
-    f.y = v[2];
-    f.py = v[3];
-    f.z = v[4];
-    bad |= lanes(!(v[5] > -0.5));
-    if (((rows | srows) >> 5 & 1)) {
-        en.pz = v[5];
-        energy_functions(en.pz, en.bq, sp, en.rel_p, en.inv_rp, en.ez, en.lez);
-        en.ir2 = en.inv_rp * en.inv_rp;
-    }
+    rad_leave(f, en, v, (rows | srows) >> 5 & 1, sp, bad);
 }
 
 // An operation of kind `code` (FO_* with its FO_RECT and FO_UCHECK bits): values v[0..] as in its

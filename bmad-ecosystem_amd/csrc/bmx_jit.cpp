@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -100,6 +101,20 @@ bool cell_ops(const HostTable &t, const Period &pd, int32_t j, std::vector<uint3
     return true;
 }
 
+// The coefficients of a radiation kick that are not zero in some cell: damp_dmat[i][j] in bit
+// 6 i + j, xfer_damp_vec[i] in bit 36 + i, stoc_mat's lower triangle by rows, and the masks of
+// rows and columns that fast_radiation's packed word has, which must be the same in every cell.
+// The kick's values in the stream: that word, ref_orb of the columns of damp_dmat in use, each
+// damping row's coefficients and xfer_damp_vec, each stochastic row's coefficients. Read row by
+// row from the packed map (fast_radiation), a kick of the usual bend waits for 8 lines one after
+// the other; these values are 24, and come with the cell's.
+struct RadTerms {
+    uint64_t damp = 0;
+    uint32_t stoc = 0, cols = 0;
+    bool energy = false;
+    bool columns(int j) const { return damp & (0x041041041ull << j) & 0xFFFFFFFFFull; }
+};
+
 // Where the values of a cell's operations lie in its stream (LatDesc::cell): lines of kFastOpLen
 // doubles, an operation's values within one line (they are in scalar registers together, and
 // the next line is loaded while the operations of one run). An aperture equal to the one before
@@ -109,6 +124,8 @@ struct CellOp {
     uint32_t code;
     int32_t at;          // first value in the stream
     int32_t ap;          // its aperture's k2 in the stream (r2 next), or -1: none
+    int32_t n = 0;       // its values
+    RadTerms rad;        // a radiation kick written out
 };
 struct CellPlan {
     std::vector<CellOp> ops;
@@ -119,6 +136,80 @@ struct CellPlan {
 const double *op_record(const HostTable &t, const Period &pd, int32_t c, const CellOp &o)
 {
     return &t.ops[(size_t)kFastOpLen * (t.fast[pd.H + c * pd.P + o.j].op0 + o.k)];
+}
+
+// The packed word of a radiation kick, and its map's values line by line in the order of RadTerms.
+uint64_t rad_word(const double *record)
+{
+    uint64_t at;
+    std::memcpy(&at, record, sizeof at);
+    return at;
+}
+
+struct RadMap {
+    double ref[6] = {}, damp[6][6] = {}, xfer[6] = {}, stoc[6][6] = {};
+};
+
+RadMap rad_map(const HostTable &t, uint64_t at)
+{
+    RadMap m;
+    const double *l = &t.rad_lines[(size_t)kFastOpLen * (at & 0xFFFFFF)];
+    std::copy(l, l + 6, m.ref);
+    for (int i = 0; i < 6; i++)
+        if (at >> (26 + i) & 1) {
+            l += kFastOpLen;
+            std::copy(l, l + 6, m.damp[i]);
+            m.xfer[i] = l[6];
+        }
+    for (int i = 0; i < 6; i++)
+        if (at >> (32 + i) & 1) {
+            l += kFastOpLen;
+            std::copy(l, l + i + 1, m.stoc[i]);
+        }
+    return m;
+}
+
+// The terms of a kick that is one in every cell with the same rows and columns; else none (n = 0).
+int32_t rad_terms(const HostTable &t, const Period &pd, const CellOp &o, RadTerms &r)
+{
+    const uint64_t masks = rad_word(op_record(t, pd, 0, o)) >> 24 & 0xFFFFF;  // edge, rows, columns
+    for (int32_t c = 0; c < pd.N; c++) {
+        const uint64_t at = rad_word(op_record(t, pd, c, o));
+        if ((at >> 24 & 0xFFFFF) != masks) return 0;
+        const RadMap m = rad_map(t, at);
+        for (int i = 0, k = 0; i < 6; i++) {
+            for (int j = 0; j < 6; j++)
+                if (m.damp[i][j] != 0) r.damp |= 1ull << (6 * i + j);
+            if (m.xfer[i] != 0) r.damp |= 1ull << (36 + i);
+            for (int j = 0; j <= i; j++, k++)
+                if (m.stoc[i][j] != 0) r.stoc |= 1u << k;
+        }
+    }
+    r.cols = masks >> 14 & 63;
+    r.energy = ((masks >> 2 | masks >> 8) >> 5) & 1;
+    int32_t n = 1 + __builtin_popcountll(r.damp) + __builtin_popcount(r.stoc);
+    for (int j = 0; j < 6; j++) n += r.columns(j);
+    return n;
+}
+
+// The values of an operation of cell c in the order of its places in the stream.
+std::vector<double> op_values(const HostTable &t, const Period &pd, int32_t c, const CellOp &o)
+{
+    const double *r = op_record(t, pd, c, o);
+    if (!o.rad.cols && !o.rad.damp) return std::vector<double>(r, r + o.n);
+    std::vector<double> v{r[0]};
+    const RadMap m = rad_map(t, rad_word(r));
+    for (int j = 0; j < 6; j++)
+        if (o.rad.columns(j)) v.push_back(m.ref[j]);
+    for (int i = 0; i < 6; i++) {
+        for (int j = 0; j < 6; j++)
+            if (o.rad.damp >> (6 * i + j) & 1) v.push_back(m.damp[i][j]);
+        if (o.rad.damp >> (36 + i) & 1) v.push_back(m.xfer[i]);
+    }
+    for (int i = 0, k = 0; i < 6; i++)
+        for (int j = 0; j <= i; j++, k++)
+            if (o.rad.stoc >> k & 1) v.push_back(m.stoc[i][j]);
+    return v;
 }
 
 CellPlan plan_cell(const HostTable &t, const Period &pd)
@@ -156,13 +247,71 @@ CellPlan plan_cell(const HostTable &t, const Period &pd)
                 o.ap = ap;
                 last = o;
             }
-            o.at = place(fast_values(kind));
+            o.n = kind == FO_RAD ? rad_terms(t, pd, o, o.rad) : 0;
+            if (o.n > 1) {  // taken one by one, over the ends of lines
+                o.at = at;
+                at += o.n;
+            } else {
+                o.rad = RadTerms{};
+                o.n = fast_values(kind);
+                o.at = place(o.n);
+            }
             p.ops.push_back(o);
         }
     }
     p.lines = (at + kFastOpLen - 1) / kFastOpLen;
     if (p.lines == 1) p.lines = 2;  // a line is loaded while the one before is in use
     return p;
+}
+
+// A radiation kick on the terms of its maps that are not zero (the arithmetic of fast_radiation with
+// the zero terms left out), each value taken as the stream brings it.
+template <class Reach, class Val>
+void write_radiation(std::ostream &b, const CellOp &o, size_t id, Reach &reach, Val &val)
+{
+    int32_t at = o.at;
+    const auto next = [&]() {
+        reach(at);
+        return val(at++);
+    };
+    const std::string k = std::to_string(id), in = "                ";
+    const std::string word = next();
+    if (o.code & FO_UCHECK) b << in << "fast_unstable(f, ef, bad);\n";
+    b << in << "const uint64_t at" << k << " = __double_as_longlong(" << word << ");\n"
+      << in << "double g" << k << "[6] = {0, 0, 0, 0, 0, 0};\n"
+      << in << "if (L.sp.rad.flags & RAD_FLUCT) rad_deviates(g" << k << ", at" << k << ", " << o.rad.cols
+      << "u, L.sp, ra);\n"
+      << in << "bad |= lanes(!(fabs(f.z) < 1e30));\n"
+      << in << "double v" << k << "[6] = {f.x, f.px, f.y, f.py, f.z, ef.pz};\n"
+      << in << "double d" << k << "[6] = {0, 0, 0, 0, 0, 0}, s" << k << ";\n";
+    for (int j = 0; j < 6; j++)
+        if (o.rad.columns(j)) {
+            const std::string v = next();
+            b << in << "d" << k << "[" << j << "] = v" << k << "[" << j << "] - " << v << ";\n";
+        }
+    // a row's sum over its terms, then coordinate i moved by it where `when` holds
+    const auto row = [&](int i, int n, uint64_t mask, const char *x, const char *when) {
+        bool any = false;
+        for (int j = 0; j < n; j++) {
+            if (!(mask >> j & 1)) continue;
+            const std::string c = next(), xj = x + k + "[" + std::to_string(j) + "]";
+            if (any) b << in << "s" << k << " = fma(" << c << ", " << xj << ", s" << k << ");\n";
+            else b << in << "s" << k << " = " << c << " * " << xj << ";\n";
+            any = true;
+        }
+        const std::string vi = "v" + k + "[" + std::to_string(i) + "]";
+        if (any) b << in << "if (" << when << ") " << vi << " = fma(L.sp.rad.scale, s" << k << ", " << vi << ");\n";
+    };
+    for (int i = 0; i < 6; i++) {
+        row(i, 6, o.rad.damp >> (6 * i) & 63, "d", "L.sp.rad.flags & RAD_DAMP");
+        if (o.rad.damp >> (36 + i) & 1) {
+            const std::string x = next(), vi = "v" + k + "[" + std::to_string(i) + "]";
+            b << in << "if ((L.sp.rad.flags & (RAD_DAMP | RAD_ZERO_AVERAGE)) == RAD_DAMP) " << vi
+              << " = fma(L.sp.rad.scale, " << x << ", " << vi << ");\n";
+        }
+    }
+    for (int i = 0, t = 0; i < 6; t += ++i) row(i, i + 1, o.rad.stoc >> t & ((1u << (i + 1)) - 1), "g", "L.sp.rad.flags & RAD_FLUCT");
+    b << in << "rad_leave(f, ef, v" << k << ", " << (o.rad.energy ? "true" : "false") << ", L.sp, bad);\n";
 }
 
 std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan, std::string &sig)
@@ -217,9 +366,9 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
             int32_t first_line = INT32_MAX, last_line = -1, ap = -1;
             for (size_t k = next_op; k < o1; k++) {
                 const CellOp &o = plan.ops[k];
-                if (fast_values(o.code & FO_KIND) > 0) {
+                if (o.n > 0) {
                     first_line = std::min(first_line, o.at / kFastOpLen);
-                    last_line = std::max(last_line, o.at / kFastOpLen);
+                    last_line = std::max(last_line, (o.at + o.n - 1) / kFastOpLen);
                 }
                 if (o.ap >= 0 && o.ap != ap) {
                     ap = o.ap;
@@ -228,6 +377,7 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
                 }
             }
             body << "            {\n"
+                 << "#pragma clang fp contract(off)\n"
                  << "                FastP f = fast_get(p);\n"
                  << "                FastE ef = en;\n"
                  << "                LaneMask bad = 0;\n"
@@ -252,7 +402,11 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
             ap = -1;
             for (size_t k = next_op; k < o1; k++) {
                 const CellOp &o = plan.ops[k];
-                const int32_t nv = fast_values(o.code & FO_KIND);
+                if (o.rad.cols || o.rad.damp) {
+                    write_radiation(body, o, k, reach, val);
+                    continue;
+                }
+                const int32_t nv = o.n;
                 if (o.ap >= 0 && o.ap != ap) {
                     ap = o.ap;
                     reach(o.ap);
@@ -286,7 +440,8 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
         key << '/' << h.kind << ',' << h.flags << ',' << h.n << ',' << h.off - t.hdr[pd.H].off << ','
             << (int)plan.fast[j] << (int)plan.open[j];
     }
-    for (const CellOp &o : plan.ops) key << ';' << o.j << ',' << o.code << ',' << o.at << ',' << o.ap;
+    for (const CellOp &o : plan.ops) key << ';' << o.j << ',' << o.code << ',' << o.at << ',' << o.ap << ',' << o.rad.damp << ',' << o.rad.stoc << ','
+            << o.rad.cols << ',' << o.rad.energy;
     if (t.rare_q) key << "/q";
     if (t.rad) key << "/r";
     sig = key.str();
@@ -401,7 +556,8 @@ int jit_specialize(int device, const HostTable &t, const JitKernels **out,
         for (const CellOp &o : plan.ops) {
             double *to = &stream[(size_t)kFastOpLen * plan.lines * c];
             const double *r = op_record(t, pd, c, o);
-            for (int i = 0; i < fast_values(o.code & FO_KIND); i++) to[o.at + i] = r[i];
+            const std::vector<double> v = op_values(t, pd, c, o);
+            std::copy(v.begin(), v.end(), to + o.at);
             if (o.ap >= 0) {
                 to[o.ap] = r[6];
                 to[o.ap + 1] = r[7];
