@@ -144,7 +144,7 @@ hipError_t enqueue_run(hipStream_t s, RunBuffers &rb, const Group *h_groups, int
     size_t all_tiles = 0;
     for (int32_t g = 0; g < n_groups; g++)
         if (h_groups[g].n_turns > 0) all_tiles += (h_groups[g].n + 63) / 64;
-    const int collect_grid = (int)std::min<size_t>((all_tiles + 3) / 4, 4096);
+    const int collect_grid = (int)std::min<size_t>((all_tiles + 3) / 4, 512);  // then several tiles per wave
     e = launch_build_tiles(s, rb.d_groups, n_groups, nullptr, 0, rb.d_tiles[1], n_tiles[1],
                            rb.d_cnt[0], tile_ctr, rb.d_goff);
     if (e == hipSuccess)

@@ -1,4 +1,4 @@
-"""Single-launch spans: the same bits as the chunked way."""
+"""Single-launch spans and the packing of live particles: the same bits as the chunked way."""
 from __future__ import annotations
 
 import numpy as np
@@ -88,3 +88,32 @@ def test_spans_in_one_launch(bmx, ctx, kind, maps):
         ctx.set_run(5, 0, 0)
         ctx.set_maps("fast")
         lat.close()
+
+
+def test_packing_of_many_groups(bmx, ctx):
+    """A batch of more tiles than the packing kernel has waves (several tiles per wave, groups that
+    begin and end inside a wave's share, particles dead on arrival): each group as by itself."""
+    E, L, T = bmx.elements, bmx.lattices, bmx.tracking
+    lat = T.Lattice(ctx, E.to_array(L.ring1(n_cells=2)))
+    rng = np.random.default_rng(5)
+    counts = np.concatenate([[1, 63, 64, 65, 0, 511, 513], rng.integers(1, 16000, 60)])
+    assert ((counts + 63) // 64).sum() > 2 * 2048
+    first = np.concatenate([[0], np.cumsum(counts)[:-1]])
+    beam = _beam(bmx, int(counts.sum()), 31)
+    print("packing", int(counts.sum()), flush=True)
+    b = T.Beam.from_host(ctx, beam)
+    batch = T.Batch(ctx, [(lat, b, int(f), int(c)) for f, c in zip(first, counts)])
+    batch.track(2)
+    ctx.synchronize()
+    got = b.download()
+    batch.close()
+    b.close()
+    for f, c in zip(first[:12], counts[:12]):
+        if c == 0:
+            continue
+        one = T.Beam.from_host(ctx, {k: v[f:f + c].copy() for k, v in beam.items()})
+        T.track_beam(ctx, lat, one, 2)
+        ctx.synchronize()
+        _same({k: v[f:f + c].copy() for k, v in got.items()}, one.download())
+        one.close()
+    lat.close()
