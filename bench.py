@@ -232,8 +232,7 @@ def main():
 
     value = passes / (total_ms * 1e-3)
     # the kernel of each step: with waves chosen automatically the library picks the 5-wave
-    # build while the live particles fill more than 1.45 rounds of the 4-wave build, then the
-    # 4-wave one (the run phase)
+    # build where the beam fills more than 1.45 rounds of the 4-wave build's resident waves
     step_waves = [int(w) for _, _, w in shapes]
     kernels = {}
     for w in step_waves:

@@ -15,6 +15,12 @@
 // each, read by one scalar load. Sums and products are written as they are to be rounded
 // (contraction is off and every fused multiply-add explicit), so that an operation gives the same
 // bits wherever it is inlined.
+//
+// What bounds the kernels made of them: large beams, the issue of vector instructions (354 for a
+// cell of 9 elements against 612 for the general maps, and 63 scalar ones against 234); few
+// particles, the chain of dependent operations and the reads of their values, one line of 64
+// bytes ahead. 901-element ring, 10 turns, general maps -> operations: 1e6 particles 18.8 -> 11.6
+// ms, 1000 particles 3.68 -> 1.34 ms with cell kernels; 150001 particles 8.8 -> 4.5 ms without.
 #pragma once
 #include <hip/hip_runtime.h>
 

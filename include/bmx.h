@@ -185,9 +185,8 @@ int32_t bmx_ctx_set_maps(bmx_ctx *ctx, int32_t form);
  * compacted between chunks; 0 = the whole call is one chunk; default 5), workgroups of the
  * persistent tracking grid (0 = as many as fit on the device at once, the default) and the
  * waves per SIMD the tracking kernel variant is compiled for at least (3, 4 or 5; 0 = chosen
- * per call: for a cell-specialised lattice 5 while the live particles fill more than 1.45
- * rounds of the 4-wave kernel's resident waves and 4 below (the run phase, from a count of the
- * live particles at the start of the call), else 5 with the fast maps, 3 with the reference
+ * per call: for a cell-specialised lattice 5 where the beam fills more than 1.45 rounds of the
+ * 4-wave kernel's resident waves and 4 below, else 5 with the fast maps, 3 with the reference
  * maps). */
 int32_t bmx_ctx_set_run(bmx_ctx *ctx, int32_t chunk_turns, int32_t grid, int32_t waves);
 /* The run shape (turns per chunk, workgroups, waves per SIMD) the context's last

@@ -178,9 +178,10 @@ def test_results_do_not_depend_on_the_wave(bmx, ctx):
                 assert np.array_equal(one[k][0:1], mixed[k][i:i + 1]), (how, i, k)
 
 
-@pytest.mark.parametrize("rows", ["none", "pz", "bend", "all"])
+@pytest.mark.parametrize("rows", ["none", "pz", "bend", "all", "coefficients", "cells"])
 def test_radiation_maps_with_zero_parts(bmx, oracle, ctx, rows):
-    """Radiation maps whose zero rows and columns the operation leaves out: damping and fluctuations of
+    """Radiation maps whose zero rows and columns the operation leaves out, the same in every cell (also
+    with single coefficients that are zero in some cells) or not ("cells"): damping and fluctuations of
     a ring of plain and gradient bends and offset quadrupoles, one turn, losses identical and
     survivors within the whole-turn bar of the restatement."""
     T = bmx.tracking
@@ -188,13 +189,18 @@ def test_radiation_maps_with_zero_parts(bmx, oracle, ctx, rows):
     e = _elements(bmx, **_apertures(bmx)["ellipse"])
     arr = E.to_array([e["drift"], e["bend"], e["quad_offset"], e["drift"], e["bend_k1"], e["sext_1"]] * 4)
     maps = R.lattice_maps(arr, bmx, damp=1e2, stoc=1e2)
-    keep = {"none": [], "pz": [5], "bend": [0, 1, 4, 5], "all": [0, 1, 2, 3, 4, 5]}[rows]
+    keep = {"none": [], "pz": [5], "bend": [0, 1, 4, 5]}.get(rows, [0, 1, 2, 3, 4, 5])
     drop = [i for i in range(6) if i not in keep]
     for f in ("damp_dmat", "stoc_mat"):
         maps[f][:, :, drop, :] = 0
         maps[f][:, :, :, drop] = 0
     maps["xfer_damp_vec"][:, :, drop] = 0
     maps["ref_orb"][...] = 1e-4
+    if rows == "coefficients":
+        maps["damp_dmat"][:12, :, 5, 0] = maps["damp_dmat"][:, :, 1, :3] = maps["xfer_damp_vec"][6:, :, 1] = 0
+        maps["stoc_mat"][6:, :, 4, 2] = maps["stoc_mat"][:, :, 3, 3] = 0
+    if rows == "cells":
+        maps["damp_dmat"][:6, :, 1, :] = maps["xfer_damp_vec"][:6, :, 1] = maps["stoc_mat"][:6, :, 2, :] = 0
     beam = _beam(bmx, 2000, 17)
     for k, s in (("x", 0.3), ("y", 0.3), ("px", 0.05), ("py", 0.05)):
         beam[k] *= s
