@@ -418,6 +418,9 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
                 body << "};\n                    fast_op<maps_rad(kRare)>(f, ef, " << o.code
                      << "u, v, k2, r2, L.sp, maps_rad(kRare), ra, bad);\n                }\n";
             }
+            // the next cell's first line is loaded behind the last one, also where no value lies in that
+            // (a cell of one line, padded to two)
+            if (carry) reach(plan.lines * kFastOpLen - 1);
             if (open) body << "                fast_unstable(f, ef, bad);\n";
             body << "                if (!bad) {\n"
                  << "                    put(p, en, f, ef);\n"

@@ -1,0 +1,101 @@
+"""Cell-specialised kernels on lattices whose cells differ in their strengths and apertures, and on
+cells of every length the kernels' value lines treat differently: against the generic kernel."""
+import numpy as np
+import pytest
+
+import parity as P
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx(bmx):
+    c = bmx.tracking.Context(0)
+    c.set_maps("fast")
+    return c
+
+
+def _track(bmx, ctx, arr, beam, special, n_turns=2):
+    T = bmx.tracking
+    lat = T.Lattice(ctx, arr)
+    if special:
+        assert lat.specialize()
+    b = T.Beam.from_host(ctx, beam)
+    T.track_beam(ctx, lat, b, n_turns, 0)
+    ctx.synchronize()
+    out = b.download()
+    b.close()
+    lat.close()
+    return out
+
+
+def _same(a, b):
+    for k in P.KEYS:
+        bits = np.int64 if a[k].dtype == np.float64 else np.int32
+        bad = np.nonzero(a[k].view(bits) != b[k].view(bits))[0]
+        assert bad.size == 0, (k, bad.size, bad[:5], a[k][bad[:5]], b[k][bad[:5]])
+
+
+# Cells by the kinds of their elements, and the values they have in the cell kernels' lines of 8: an
+# aperture (2, here the same in every cell) and 1 for a drift, 2 for a kicker, 3 for a quadrupole or a
+# sextupole, 6 for a bend.
+CELLS = {
+    "q": 5, "b": 8, "dq": 6, "dk": 5, "kq": 7, "qs": 8, "ddq": 7,  # one line
+    "qds": 9, "dqdb": 15, "qsbdd": 16, "dqsdbdqsb": 33,            # several
+    "dqkdsqbdqskdqsbdqdb": 70,                                     # several runs of operations
+}
+
+
+def _cells(bmx, kinds, seed, apertures=False):
+    """24 cells (8 long ones) of the given kinds, each element with strengths of its own (the sign of
+    k1 changes from quadrupole to quadrupole and from cell to cell) and all of them on operations;
+    apertures: half-axes that change from cell to cell as well."""
+    E = bmx.elements
+    p0c, et = bmx.lattices.reference()
+    rng = np.random.default_rng(seed)
+    out = []
+    for c in range(24 if len(kinds) < 10 else 8):
+        s = rng.uniform(0.5, 1.0, len(kinds))
+        for i, (kind, w) in enumerate(zip(kinds, s)):
+            sign = (-1) ** (c + kinds[:i].count("q"))
+            ap = dict(x_limit=0.02 * (w if apertures else 1.0), y_limit=0.02, aperture_type=E.APERTURE_ELLIPTICAL)
+            mk = lambda key, **kw: E.make_element(key, p0c, et, **kw, **ap)  # noqa: E731, B023
+            out.append({
+                "d": lambda: mk(E.DRIFT, l=0.4 * w),
+                "q": lambda: mk(E.QUADRUPOLE, l=0.3, k1=sign * 0.5 * w),
+                "s": lambda: mk(E.SEXTUPOLE, l=0.2, k2=sign * 2.0 * w, num_steps=1),
+                "k": lambda: mk(E.KICKER, hkick=1e-6 * w, vkick=-1e-6 * w),
+                "b": lambda: mk(E.SBEND, l=1.0, g=0.016 + 0.005 * w),
+            }[kind]())
+    return out
+
+
+@pytest.mark.parametrize("kinds, ends", [(k, False) for k in CELLS] +
+                         [(k, True) for k in ("q", "dq", "qds", "dqkdsqbdqskdqsbdqdb")])
+def test_cells_of_their_own_strengths(bmx, ctx, kinds, ends):
+    """A ring of cells with strengths of their own, alone or with a head and a tail of other
+    elements: the cell kernel and the generic one give the same bits, with lost particles among
+    the others and without."""
+    E = bmx.elements
+    p0c, et = bmx.lattices.reference()
+    eles = _cells(bmx, kinds, 11)
+    if ends:
+        mk = lambda **kw: E.make_element(E.QUADRUPOLE, p0c, et, l=0.2, tilt=0.3, **kw)  # noqa: E731
+        eles = [mk(k1=0.02 * (-1) ** i) for i in range(len(kinds))] + eles + [mk(k1=-0.02)]
+    arr = E.to_array(eles)
+    for scale in (1.0, 40.0):
+        beam = P.random_beam(bmx, 1000, 3, scale=scale, pz_sigma=1e-3)
+        print(f"cells {kinds} ends {ends} scale {scale}", flush=True)
+        want = _track(bmx, ctx, arr, beam, False)
+        assert (want["state"] == 1).sum() > 50
+        if scale > 1 and "q" in kinds:
+            assert (want["state"] != 1).sum() > 0
+        _same(_track(bmx, ctx, arr, beam, True), want)
+
+
+@pytest.mark.parametrize("kinds", ["q", "dq", "dqdb", "dqkdsqbdqskdqsbdqdb"])
+def test_apertures_that_change_from_cell_to_cell(bmx, ctx, kinds):
+    arr = bmx.elements.to_array(_cells(bmx, kinds, 12, apertures=True))
+    beam = P.random_beam(bmx, 1000, 4, scale=25.0, pz_sigma=1e-3)
+    print(f"cell apertures {kinds}", flush=True)
+    _same(_track(bmx, ctx, arr, beam, True), _track(bmx, ctx, arr, beam, False))
