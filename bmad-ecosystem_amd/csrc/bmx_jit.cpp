@@ -314,13 +314,47 @@ void write_radiation(std::ostream &b, const CellOp &o, size_t id, Reach &reach, 
     b << in << "rad_leave(f, ef, v" << k << ", " << (o.rad.energy ? "true" : "false") << ", L.sp, bad);\n";
 }
 
-std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan, std::string &sig)
+// The map set the cell kernels of a lattice carry on their rare path, by all its elements: those of
+// the head and the tail are tracked by these kernels too.
+struct CellMaps {
+    bool q_kinds = false;  // stepped quadrupoles or general bends
+    const char *rare;
+};
+
+CellMaps cell_maps(const HostTable &t)
 {
-    bool q_kinds = false;  // the lattice holds stepped quadrupoles or general bends
-    for (const EleHdr &h : t.hdr) q_kinds |= h.kind == K_QMULT || h.kind == K_BMULT;
-    std::ostringstream body, key;
-    key << pd.H << ':' << pd.P << ':' << pd.N << ':' << pd.S << ':' << t.hdr.size() << ':'
-        << t.hdr[pd.H].off;
+    CellMaps m;
+    for (const EleHdr &h : t.hdr) m.q_kinds |= h.kind == K_QMULT || h.kind == K_BMULT;
+    m.rare = t.rad ? (m.q_kinds ? "MAPS_RARE_QR" : "MAPS_RARE_R") : t.rare_q ? "MAPS_RARE_Q" : "MAPS_RARE";
+    return m;
+}
+
+// All that the kernels' source is made from, and so their key in the cache. Taken without writing
+// the source, which a lattice whose kernels are there does not need.
+std::string signature(const HostTable &t, const Period &pd, const CellPlan &plan, const CellMaps &maps)
+{
+    std::string key = maps.rare;
+    const auto put = [&](auto v) { key.append((const char *)&v, sizeof v); };
+    for (const int32_t v : {pd.H, pd.P, pd.N, pd.S, (int32_t)t.hdr.size(), t.hdr[pd.H].off, (int32_t)maps.q_kinds}) put(v);
+    for (int32_t j = 0; j < pd.P; j++) {
+        const EleHdr &h = t.hdr[pd.H + j];
+        for (const int32_t v : {h.kind, h.flags, h.n, h.off - t.hdr[pd.H].off}) put(v);
+        put(plan.fast[j]);
+        put(plan.open[j]);
+    }
+    for (const CellOp &o : plan.ops) {
+        for (const int32_t v : {o.j, o.k, (int32_t)o.code, o.at, o.ap, o.n}) put(v);
+        put(o.rad.damp);
+        put(o.rad.stoc);
+        put(o.rad.cols);
+        put(o.rad.energy);
+    }
+    return key;
+}
+
+std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan, const CellMaps &maps)
+{
+    std::ostringstream body;
     // The cell in segments: runs of at most kFastBlockOps operations (bmx_fast.hpp), and its other
     // elements. A segment that leaves something to the general maps (elements of theirs, or the lanes
     // a run refused) leaves the cell loop with its element range and the next segment's
@@ -438,16 +472,6 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
         next_op = o1;
         j = j1;
     }
-    for (int32_t j = 0; j < pd.P; j++) {
-        const EleHdr &h = t.hdr[pd.H + j];
-        key << '/' << h.kind << ',' << h.flags << ',' << h.n << ',' << h.off - t.hdr[pd.H].off << ','
-            << (int)plan.fast[j] << (int)plan.open[j];
-    }
-    for (const CellOp &o : plan.ops) key << ';' << o.j << ',' << o.code << ',' << o.at << ',' << o.ap << ',' << o.rad.damp << ',' << o.rad.stoc << ','
-            << o.rad.cols << ',' << o.rad.energy;
-    if (t.rare_q) key << "/q";
-    if (t.rad) key << "/r";
-    sig = key.str();
     std::ostringstream s;
     s << "#include <stdint.h>\n"
       << bmx_jit_src_table << '\n'
@@ -456,8 +480,7 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
       << bmx_jit_src_tiles << '\n'
       << "namespace bmx {\n"
       << "struct CellTurn {\n"
-      << "    static constexpr int kRare = "
-      << (t.rad ? (q_kinds ? "MAPS_RARE_QR" : "MAPS_RARE_R") : t.rare_q ? "MAPS_RARE_Q" : "MAPS_RARE") << ";\n"
+      << "    static constexpr int kRare = " << maps.rare << ";\n"
       << "    __device__ __forceinline__ static void put(Particle &p, FastE &en, const FastP &f, const FastE &ef)\n"
       << "    {\n"
       << "        fast_put(p, f);\n"
@@ -531,7 +554,7 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
     // the stepped-element map sets only for its radiation kicks gets the variants asked for
     for (int w = 3; w <= 5; w++)
         s << "extern \"C\" __global__ void __launch_bounds__(bmx::kBlock) "
-          << "__attribute__((amdgpu_waves_per_eu(" << (q_kinds ? 2 : w) << "))) bmx_cell_tiles_" << w << args
+          << "__attribute__((amdgpu_waves_per_eu(" << (maps.q_kinds ? 2 : w) << "))) bmx_cell_tiles_" << w << args
           << "\n{\n    bmx::track_tiles<true, bmx::CellTurn>(g, t, nt, pi, po, ps, co, tc, off, K, w);\n}\n";
     return s.str();
 }
@@ -550,9 +573,8 @@ int jit_specialize(int device, const HostTable &t, const JitKernels **out,
         err = "no repeated cell covering three quarters of the lattice";
         return BMX_ERR_UNSUPPORTED;
     }
-    std::string sig;
     const CellPlan plan = plan_cell(t, pd);
-    const std::string src = generate(t, pd, plan, sig);
+    const CellMaps maps = cell_maps(t);
     // the cells' values in the plan's places, and a line that the last cell's loads may reach
     stream.assign((size_t)kFastOpLen * ((size_t)plan.lines * pd.N + 1), 0.0);
     for (int32_t c = 0; c < pd.N; c++)
@@ -567,11 +589,12 @@ int jit_specialize(int device, const HostTable &t, const JitKernels **out,
             }
         }
     std::lock_guard<std::mutex> lock(g_mutex);
-    auto &slot = g_cache[{device, sig}];
+    auto &slot = g_cache[{device, signature(t, pd, plan, maps)}];
     if (slot) {
         *out = slot.get();
         return BMX_OK;
     }
+    const std::string src = generate(t, pd, plan, maps);
     hiprtcProgram prog;
     if (hiprtcCreateProgram(&prog, src.c_str(), "bmx_cell.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS) {
         err = "hiprtcCreateProgram failed";

@@ -99,3 +99,43 @@ def test_apertures_that_change_from_cell_to_cell(bmx, ctx, kinds):
     beam = P.random_beam(bmx, 1000, 4, scale=25.0, pz_sigma=1e-3)
     print(f"cell apertures {kinds}", flush=True)
     _same(_track(bmx, ctx, arr, beam, True), _track(bmx, ctx, arr, beam, False))
+
+
+@pytest.mark.parametrize("general_first", [False, True])
+def test_radiating_lattices_of_the_same_cells(bmx, ctx, general_first):
+    """Two radiating lattices of the same cells and length, the last element a plain bend in one and a
+    bend with a sextupole part in the other, specialised one after the other: each as on the
+    generic kernel (losses identical, survivors within the per-element bar, 1e-12, for each element
+    passed: the general maps are contracted by the compiler for each kernel)."""
+    E, T = bmx.elements, bmx.tracking
+    p0c, et = bmx.lattices.reference()
+    mk = lambda key, **kw: E.make_element(key, p0c, et, **kw, x_limit=0.02, y_limit=0.02)  # noqa: E731
+    cells = 9 + general_first  # kernels of its own for each order
+    cell = [mk(E.DRIFT, l=0.5), mk(E.SBEND, l=1.0, g=0.02), mk(E.QUADRUPOLE, l=0.3, k1=0.05)]
+    ends = {False: mk(E.SBEND, l=1.0, g=0.02), True: mk(E.SBEND, l=1.0, g=0.02, b_pole={2: 20.0}, num_steps=2)}
+    beam = P.random_beam(bmx, 500, 8, scale=3.0, pz_sigma=1e-3)
+    held = []
+    for general in (general_first, not general_first):
+        arr = E.to_array(cell * cells + [ends[general]])
+        maps = T.rad_maps(len(arr))
+        for i in np.nonzero(arr["key"] == E.SBEND)[0]:
+            maps["damp_dmat"][i, :, 5, 5] = -1e-5
+            maps["stoc_mat"][i, :, 5, 5] = 1e-6
+        outs = []
+        for special in (False, True):
+            lat = T.Lattice(ctx, arr, rad_maps=maps, rad=T.rad_config(True, True, seed=7))
+            held.append(lat)
+            if special:
+                assert lat.specialize()
+            b = T.Beam.from_host(ctx, beam)
+            print(f"radiating lattices, general {general}, special {special}", flush=True)
+            T.track_beam(ctx, lat, b, 2, 0)
+            ctx.synchronize()
+            outs.append(b.download())
+            b.close()
+        assert P.loss_mismatch(outs[1], outs[0]).size == 0, general
+        alive = outs[0]["state"] == 1
+        assert alive.sum() > 50
+        assert P.rel_err(outs[1], outs[0], alive) <= 1e-12 * 2 * len(arr), general
+    for lat in held:
+        lat.close()
