@@ -190,7 +190,10 @@ int32_t bmx_lattice_set_radiation(bmx_lattice *L, const bmx_rad_config *config)
     if (!L || !config || config->reserved != 0 || !std::isfinite(config->synch_rad_scale))
         return set_error(BMX_ERR_ARG, "bmx_lattice_set_radiation: bad argument");
     L->host.sp.rad = rad_settings(*config);
-    L->desc.sp.rad = L->host.sp.rad;
+    {
+        std::lock_guard<std::mutex> lock(L->mu);
+        L->desc.sp.rad = L->host.sp.rad;
+    }
     // runs take the descriptor by value when they are queued; those queued before keep theirs
     hipSetDevice(L->device);
     HIP_TRY(hipStreamSynchronize(L->ctx->stream), "bmx_lattice_set_radiation: sync");
@@ -292,8 +295,9 @@ int32_t bmx_lattice_specialize(bmx_lattice *L)
             return hip_fail(e, "bmx_lattice_specialize: cell values");
         }
         L->d_cell = d;
-        L->desc.cell = d;
     }
+    std::lock_guard<std::mutex> lock(L->mu);
+    L->desc.cell = L->d_cell;
     L->jit = j;
     return BMX_OK;
 }

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -193,10 +194,22 @@ struct bmx_lattice {
     bmx_ctx *ctx = nullptr;
     int device = 0;
     bmx::HostTable host;
-    char *d_table = nullptr;          // every device array of the table, and its descriptor
+    char *d_table = nullptr;          // every device array of the table
     double *d_cell = nullptr;         // operation values of the cell kernels (specialised)
     bmx::LatDesc desc{};              // device pointers inside
     const bmx::JitKernels *jit = nullptr;  // set by bmx_lattice_specialize
+    // A server's thread reads desc and jit while the caller's may specialise the lattice or change its
+    // radiation settings: the changes are made, and the server's copies taken, under this lock.
+    mutable std::mutex mu;
+    struct View {
+        bmx::LatDesc desc;
+        const bmx::JitKernels *jit;
+    };
+    View view() const
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        return {desc, jit};
+    }
 };
 
 struct bmx_beam {

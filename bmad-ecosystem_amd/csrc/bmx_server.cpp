@@ -253,10 +253,15 @@ void bmx_server::run()
             groups.resize(running.size());
             int32_t max_turns = 0;
             size_t tiles = 0;
+            // the cell-specialised kernels when every request of this chunk tracks through
+            // lattices that share them, from the same view of a lattice as its cell values
+            const JitKernels *j = nullptr;
             for (size_t i = 0; i < running.size(); i++) {
                 Request *r = running[i];
                 Group &g = groups[i];
-                g.lat = r->lat->desc;
+                const bmx_lattice::View v = r->lat->view();
+                j = i == 0 || v.jit == j ? v.jit : nullptr;
+                g.lat = v.desc;
                 g.b = at(r->off);
                 g.n = (uint32_t)r->n;
                 g.list_off = (uint32_t)r->off;
@@ -267,18 +272,11 @@ void bmx_server::run()
                 max_turns = std::max(max_turns, g.n_turns);
                 tiles += (size_t)(r->n + 63) / 64;
             }
-            // the cell-specialised kernels when every request of this chunk tracks through
-            // lattices that share them
             RunConfig run = cfg;
-            if (cfg.fast) {
-                const JitKernels *j = running[0]->lat->jit;
-                for (Request *r : running)
-                    if (r->lat->jit != j) j = nullptr;
-                if (j) {
-                    run.jit = j;
-                    if (waves_auto) run.waves = default_waves(true, j);
-                    run.grid = default_grid(device, true, run.waves, j);
-                }
+            if (cfg.fast && j) {
+                run.jit = j;
+                if (waves_auto) run.waves = default_waves(true, j);
+                run.grid = default_grid(device, true, run.waves, j);
             }
             t_launch = now_ns();
             if (e == hipSuccess) e = rb.reserve(groups.size(), (size_t)capacity, tiles + 1);
