@@ -1,6 +1,7 @@
 // C-ABI of the tracking library (declared in include/bmx.h).
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -30,16 +31,16 @@ static int hip_fail(hipError_t e, const char *what)
         if (_e != hipSuccess) return bmx::hip_fail(_e, what); \
     } while (0)
 
-// Equal kernel arguments: the same device arrays and values (a captured launch holds them).
-static bool same_launch(const LatDesc &a, const LatDesc &b)
+// What a captured launch holds of a lattice: its device arrays and, by value, its descriptor. Arrays
+// of a lattice that is gone can come back at the same addresses with another one's contents, so
+// a launch is known by a number that no other lattice has, nor the same one with other settings.
+static uint64_t new_serial()
 {
-    return a.hdr == b.hdr && a.prm == b.prm && a.ops == b.ops && a.n_ele == b.n_ele && a.sp.mc2 == b.sp.mc2 &&
-           a.sp.p0c == b.sp.p0c && a.sp.mc2_sq == b.sp.mc2_sq && a.sp.beta0 == b.sp.beta0 &&
-           a.sp.me2 == b.sp.me2 && a.sp.lez_f == b.sp.lez_f && a.sp.lez_thr == b.sp.lez_thr &&
-           a.sp.rad.scale == b.sp.rad.scale && a.sp.rad.flags == b.sp.rad.flags &&
-           a.sp.rad.key0 == b.sp.rad.key0 && a.sp.rad.key1 == b.sp.rad.key1;
+    static std::atomic<uint64_t> last{0};
+    return ++last;
 }
 
+// The same device arrays.
 static bool same_launch(const BeamPtrs &a, const BeamPtrs &b)
 {
     return a.x == b.x && a.px == b.px && a.y == b.y && a.py == b.py && a.z == b.z && a.pz == b.pz &&
@@ -194,6 +195,7 @@ int32_t bmx_lattice_set_radiation(bmx_lattice *L, const bmx_rad_config *config)
         std::lock_guard<std::mutex> lock(L->mu);
         L->desc.sp.rad = L->host.sp.rad;
     }
+    L->serial = new_serial();
     // runs take the descriptor by value when they are queued; those queued before keep theirs
     hipSetDevice(L->device);
     HIP_TRY(hipStreamSynchronize(L->ctx->stream), "bmx_lattice_set_radiation: sync");
@@ -246,6 +248,7 @@ int32_t lattice_upload(bmx_ctx *ctx, HostTable &&table, bmx_lattice **out)
     L->desc.n_ele = (int32_t)t.hdr.size();
     L->desc.rare_q = t.rare_q ? (t.rad ? 2 : 1) : 0;
     L->desc.sp = t.sp;
+    L->serial = new_serial();
     *out = L;
     return BMX_OK;
 }
@@ -592,7 +595,7 @@ int32_t bmx_track_turns_plain(bmx_ctx *ctx, const bmx_lattice *L, bmx_beam *B, i
     // lattice, beam and maps) and replayed once per turn; the launches read the turn index from
     // device memory, which the graph's last node advances.
     bmx_ctx::PlainGraph &pg = ctx->plain;
-    if (!pg.exec || !same_launch(pg.lat, L->desc) || !same_launch(pg.beam, B->d) || pg.n != B->n ||
+    if (!pg.exec || pg.lat != L->serial || !same_launch(pg.beam, B->d) || pg.n != B->n ||
         pg.fast != ctx->fast_maps) {
         if (pg.exec) {
             // replays of the previous graph may still be queued
@@ -615,7 +618,7 @@ int32_t bmx_track_turns_plain(bmx_ctx *ctx, const bmx_lattice *L, bmx_beam *B, i
             pg.exec = nullptr;
             return hip_fail(e, "bmx_track_turns_plain: turn graph");
         }
-        pg.lat = L->desc;
+        pg.lat = L->serial;
         pg.beam = B->d;
         pg.n = B->n;
         pg.fast = ctx->fast_maps;

@@ -182,8 +182,8 @@ struct bmx_ctx {
     // the plain path's turn of element launches, captured once per (lattice, beam, maps) and
     // replayed for every turn
     struct PlainGraph {
-        bmx::LatDesc lat{};    // the kernel arguments the graph was captured with
-        bmx::BeamPtrs beam{};
+        uint64_t lat = 0;      // the lattice the graph was captured with (bmx_lattice::serial)
+        bmx::BeamPtrs beam{};  // and the beam's arrays
         int64_t n = -1;
         bool fast = true;
         hipGraphExec_t exec = nullptr;
@@ -197,6 +197,7 @@ struct bmx_lattice {
     char *d_table = nullptr;          // every device array of the table
     double *d_cell = nullptr;         // operation values of the cell kernels (specialised)
     bmx::LatDesc desc{};              // device pointers inside
+    uint64_t serial = 0;              // never the same for two lattices or two radiation settings of one
     const bmx::JitKernels *jit = nullptr;  // set by bmx_lattice_specialize
     // A server's thread reads desc and jit while the caller's may specialise the lattice or change its
     // radiation settings: the changes are made, and the server's copies taken, under this lock.

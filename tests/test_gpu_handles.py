@@ -42,3 +42,45 @@ def test_specialising_lattices_that_are_served(bmx, ctx):
     server.close()
     for lat in lats:
         lat.close()
+
+
+def test_plain_turns_of_replaced_lattices(bmx, ctx):
+    """The plain path keeps a captured turn from call to call: lattices of equal length and different
+    maps, each made after the one before was destroyed (their tables may come back at the same
+    addresses), and radiation settings changed between calls, each as on the persistent kernel
+    (losses identical, survivors within the per-element bar, 1e-12, for each element passed)."""
+    E, T = bmx.elements, bmx.tracking
+    p0c, et = bmx.lattices.reference()
+    mk = lambda key, **kw: E.make_element(key, p0c, et, **kw, x_limit=0.02, y_limit=0.02)  # noqa: E731
+    d, b = mk(E.DRIFT, l=0.5), mk(E.SBEND, l=1.0, g=0.02)
+    q = mk(E.QUADRUPOLE, l=0.3, k1=0.2)
+    q2 = mk(E.QUADRUPOLE, l=0.3, k1=-0.2, b_pole={2: 2.0}, num_steps=2)
+    off = mk(E.QUADRUPOLE, l=0.3, k1=-0.2, x_offset=1e-4, tilt=0.1)
+    beam = P.random_beam(bmx, 300, 6, scale=10.0, pz_sigma=1e-3)
+    gb = T.Beam.from_host(ctx, beam)
+    for round_ in range(2):
+        for name, cell, rad in (("plain", [d, q, d, b], False), ("stepped", [d, q2, d, b], False),
+                                ("radiating", [d, q, d, b], True), ("offset", [d, off, d, b], False),
+                                ("stepped radiating", [d, q2, d, b], True), ("drifts", [d] * 4, False)):
+            arr = E.to_array(cell * 6)
+            maps = T.rad_maps(len(arr)) if rad else None
+            if rad:
+                maps["damp_dmat"][3::4, :, 5, 5] = -1e-4
+                maps["stoc_mat"][3::4, :, 5, 5] = 1e-5
+            lat = T.Lattice(ctx, arr, rad_maps=maps, rad=T.rad_config(True, True, seed=3) if rad else None)
+            for seed in ((3, 4) if rad else (0,)):
+                if seed == 4:
+                    lat.set_radiation(T.rad_config(True, True, seed=seed))
+                print(f"plain turns {name} round {round_} seed {seed}", flush=True)
+                outs = []
+                for track in (T.track_beam_plain, T.track_beam):
+                    gb.upload(beam)
+                    track(ctx, lat, gb, 2, 0)
+                    ctx.synchronize()
+                    outs.append(gb.download())
+                assert P.loss_mismatch(*outs).size == 0, name
+                alive = outs[1]["state"] == 1
+                assert alive.sum() > 50
+                assert P.rel_err(outs[0], outs[1], alive) <= 1e-12 * 2 * len(arr), name
+            lat.close()
+    gb.close()
