@@ -78,27 +78,27 @@ bool find_period(const HostTable &t, Period &out)
     return false;
 }
 
-// The operations of the element at cell position j when every cell has the same ones there
-// (their tests on entering united), else false: the general maps take it.
-bool cell_ops(const HostTable &t, const Period &pd, int32_t j, std::vector<uint32_t> &codes, bool &open)
+// How the cell kernels track the element at a cell position: on its operations where every cell has
+// the same ones there (their tests on entering united), by the general maps written out where no cell has
+// any, and by the tables where the cells differ.
+enum CellForm : char { CELL_GENERAL = 0, CELL_OPS = 1, CELL_TABLE = 2 };
+CellForm cell_ops(const HostTable &t, const Period &pd, int32_t j, std::vector<uint32_t> &codes, bool &open)
 {
-    codes.clear();
     open = false;
     const int32_t n = t.fast[pd.H + j].n_ops;
-    if (n <= 0) return false;
     codes.assign(n, 0);
     for (int32_t c = 0; c < pd.N; c++) {
         const int32_t i = pd.H + c * pd.P + j;
         const FastEle &fe = t.fast[i];
-        if (fe.n_ops != n) return false;
+        if (fe.n_ops != n) return CELL_TABLE;
         open |= t.fast_open[i] != 0;
         for (int32_t k = 0; k < n; k++) {
             const uint32_t v = (uint32_t)(fe.codes[k >> 3] >> (8 * (k & 7)) & 255);
-            if (c > 0 && (v & ~FO_UCHECK) != (codes[k] & ~FO_UCHECK)) return false;
+            if (c > 0 && (v & ~FO_UCHECK) != (codes[k] & ~FO_UCHECK)) return CELL_TABLE;
             codes[k] |= v;
         }
     }
-    return true;
+    return n > 0 ? CELL_OPS : CELL_GENERAL;
 }
 
 // The coefficients of a radiation kick that are not zero in some cell: damp_dmat[i][j] in bit
@@ -129,7 +129,7 @@ struct CellOp {
 };
 struct CellPlan {
     std::vector<CellOp> ops;
-    std::vector<char> fast, open;  // per element: on operations; the last leaves px, py untested
+    std::vector<char> fast, open;  // per element: CellForm; its last operation leaves px, py untested
     int32_t lines = 0;
 };
 
@@ -228,11 +228,11 @@ CellPlan plan_cell(const HostTable &t, const Period &pd)
     for (int32_t j = 0; j < pd.P; j++) {
         std::vector<uint32_t> codes;
         bool open;
-        if (!cell_ops(t, pd, j, codes, open)) {
+        p.fast[j] = cell_ops(t, pd, j, codes, open);
+        if (p.fast[j] != CELL_OPS) {
             ap = -1;
             continue;
         }
-        p.fast[j] = 1;
         p.open[j] = open;
         for (size_t k = 0; k < codes.size(); k++) {
             CellOp o{j, (int32_t)k, codes[k], 0, -1};
@@ -356,14 +356,21 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
 {
     std::ostringstream body;
     // The cell in segments: runs of at most kFastBlockOps operations (bmx_fast.hpp), and its other
-    // elements. A segment that leaves something to the general maps (elements of theirs, or the lanes
-    // a run refused) leaves the cell loop with its element range and the next segment's
-    // number; the general maps' one call site takes the range and the loop is entered again there.
+    // elements, whose general maps are written out with their kinds and flags as constants. A run that
+    // refuses lanes leaves the cell loop with its element range and the next segment's
+    // number; the table-driven loop's one call site takes them through the range and the cell
+    // loop is entered again there. Lanes that an element of the general maps loses leave it too.
+    // (Left to the table-driven loop as well, those elements took 1.3 to 2.5 times as long: a
+    // stepped quadrupole in each cell, 100000 particles, 200 elements, 3 turns 1555 us against
+    // 473, octupoles 801 against 342, bends beyond 0.1 rad 872 against 495.)
     size_t next_op = 0;
+    // A cell with such elements also keeps a wave with a lane near the zero orbit, which a cell of
+    // operations alone leaves to the tables: its runs have the semi-linear bend.
+    const bool mixed = std::count(plan.fast.begin(), plan.fast.end(), CELL_GENERAL) > 0;
     // One run that is the whole cell loads the next cell's first line behind its last one and
     // carries it over; otherwise each run loads its own first line.
     bool carry = (int32_t)plan.ops.size() <= kFastBlockOps && !plan.ops.empty();
-    for (int32_t j = 0; j < pd.P; j++) carry = carry && plan.fast[j];
+    for (int32_t j = 0; j < pd.P; j++) carry = carry && plan.fast[j] == CELL_OPS;
     int32_t n_seg = 0;
     auto leave = [&](int32_t j0, int32_t j1) {
         std::ostringstream r;
@@ -374,9 +381,31 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
     };
     for (int32_t j = 0; j < pd.P;) {
         body << "            case " << n_seg << ":\n";
-        if (!plan.fast[j]) {
+        if (plan.fast[j] == CELL_GENERAL) {
+            int32_t j1 = j;
+            bool energy = false;
+            for (; j1 < pd.P && plan.fast[j1] == CELL_GENERAL; j1++) {
+                const EleHdr &h = t.hdr[pd.H + j1];
+                // the rare set where the table-driven loops take it; elsewhere pz cannot change
+                const bool rare = h.kind == K_RF || (h.flags & (F_OFFSET | F_APE_MOMENTUM | F_RARE_MAP));
+                energy |= rare;
+                body << "                if (p.state == ST_ALIVE)\n"
+                     << "                    track_element<true, " << (rare ? "kRare" : "MAPS_NO_RF") << ">(p, EleRef{" << h.kind
+                     << ", " << h.flags << ", " << h.n << ", " << h.off - t.hdr[pd.H].off << "}, base, L.sp, true, eb + "
+                     << j1 + 1 << ", t_abs);\n";
+            }
+            if (energy)
+                body << "                en = fast_energy(p, L.sp);\n"
+                     << "                near = !maps_rad(kRare) && near_zero<kRare>(p);\n";
+            body << "                who = lanes(p.state != ST_ALIVE);\n"
+                 << "                if (who) { " << leave(j1, j1) << " }\n";
+            n_seg++;
+            j = j1;
+            continue;
+        }
+        if (plan.fast[j] == CELL_TABLE) {
             int32_t j1 = j + 1;
-            while (j1 < pd.P && !plan.fast[j1]) j1++;
+            while (j1 < pd.P && plan.fast[j1] == CELL_TABLE) j1++;
             body << "                who = ~(LaneMask)0;\n                " << leave(j, j1) << '\n';
             n_seg++;
             j = j1;
@@ -386,7 +415,7 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
         int32_t j1 = j, n = 0;
         size_t o1 = next_op;
         bool open = false;
-        while (j1 < pd.P && plan.fast[j1]) {
+        while (j1 < pd.P && plan.fast[j1] == CELL_OPS) {
             size_t o = o1;
             while (o < plan.ops.size() && plan.ops[o].j == j1) o++;
             if (n > 0 && n + (int32_t)(o - o1) > kFastBlockOps) break;
@@ -450,7 +479,7 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
                 body << "                {\n                    const double v[6] = {";
                 for (int32_t i = 0; i < 6; i++) body << (i ? ", " : "") << (i < nv ? val(o.at + i) : "0.0");
                 body << "};\n                    fast_op<maps_rad(kRare)>(f, ef, " << o.code
-                     << "u, v, k2, r2, L.sp, maps_rad(kRare), ra, bad);\n                }\n";
+                     << "u, v, k2, r2, L.sp, maps_rad(kRare)" << (mixed ? " || near" : "") << ", ra, bad);\n                }\n";
             }
             // the next cell's first line is loaded behind the last one, also where no value lies in that
             // (a cell of one line, padded to two)
@@ -507,27 +536,31 @@ std::string generate(const HostTable &t, const Period &pd, const CellPlan &plan,
       << "            if (e0 < e1) {\n"
       << "                if (this_lane(who)) {\n"
       << "                    track_range_fast<kRare>(p, en, L, e0, e1, t_abs, stepwise);\n"
-      << "                }\n"
-      << "                if (p.state != ST_ALIVE) break;\n"
+      << "                }\n";
+    // (lanes lost in an element written out come here with an empty range)
+    if (mixed) s << "            }\n            {\n";
+    s << "                if (p.state != ST_ALIVE) break;\n"
       << "                near = !maps_rad(kRare) && near_zero<kRare>(p);\n"
       << "            }\n"
-      << "            if (done) break;\n"
-      // a wave with a lane near the zero orbit goes on by the tables, which have the semi-linear bend
-      << "            if (near) {\n"
-      << "                e0 = e1;\n"
-      << "                e1 = L.n_ele;\n"
-      << "                who = ~(LaneMask)0;\n"
-      << "                stepwise = false;\n"
-      << "                done = true;\n"
-      << "                continue;\n"
-      << "            }\n"
-      << "            stepwise = true;\n"
+      << "            if (done) break;\n";
+    // a wave with a lane near the zero orbit goes on by the tables, which have the semi-linear bend
+    if (!mixed)
+        s << "            if (near) {\n"
+          << "                e0 = e1;\n"
+          << "                e1 = L.n_ele;\n"
+          << "                who = ~(LaneMask)0;\n"
+          << "                stepwise = false;\n"
+          << "                done = true;\n"
+          << "                continue;\n"
+          << "            }\n";
+    s << "            stepwise = true;\n"
       << "            who = 0;\n";
     if (carry) s << "            OpVec l0 = load_op(cells + c * " << plan.lines * kFastOpLen << ");\n";
     s << "            for (; c < " << pd.N << "; ++c) {\n"
       << "                c = __builtin_amdgcn_readfirstlane(c);\n"
       << "                const CP cell = cells + c * " << plan.lines * kFastOpLen << ";\n"
       << "                const int32_t eb = " << pd.H << " + c * " << pd.P << ";\n"
+      << "                const CP base = (CP)L.prm + (" << t.hdr[pd.H].off << " + c * " << pd.S << ");\n"
       << "                switch (seg) {\n"
       << body.str()
       << "                default: seg = 0;\n"

@@ -139,3 +139,65 @@ def test_radiating_lattices_of_the_same_cells(bmx, ctx, general_first):
         assert P.rel_err(outs[1], outs[0], alive) <= 1e-12 * 2 * len(arr), general
     for lat in held:
         lat.close()
+
+
+def _general(bmx, kind):
+    E = bmx.elements
+    p0c, et = bmx.lattices.reference()
+    mk = lambda key, **kw: E.make_element(key, p0c, et, **kw, x_limit=0.02, y_limit=0.02)  # noqa: E731
+    return {
+        "octupole": lambda w: mk(E.OCTUPOLE, l=0.2, k3=50.0 * w),
+        "long bend": lambda w: mk(E.SBEND, l=2.0, g=0.06 + 0.01 * w),
+        "pitch": lambda w: mk(E.QUADRUPOLE, l=0.3, k1=0.03 * w, x_pitch=1e-4),
+        "stepped": lambda w: mk(E.QUADRUPOLE, l=0.3, k1=0.03 * w, b_pole={2: 1.0}, num_steps=2),
+        "general bend": lambda w: mk(E.SBEND, l=1.0, g=0.02, e1=0.02 * w, k1=1e-3, b_pole={2: 0.1}, num_steps=2),
+        "multipole": lambda w: mk(E.MULTIPOLE, knl={2: 1.0 * w, 3: 5.0}),
+        "cavity": lambda w: mk(E.RFCAVITY, l=0.5, voltage=1e6 * w, rf_frequency=500e6),
+    }[kind]
+
+
+@pytest.mark.parametrize("kind", ["octupole", "long bend", "pitch", "stepped", "general bend", "multipole", "cavity"])
+def test_cells_with_elements_of_the_general_maps(bmx, ctx, kind):
+    """Cells of operations with elements of the general maps among them, first, last and next to each
+    other, of strengths of their own: losses as on the generic kernel, survivors within the
+    per-element bar, 1e-12, for each element passed (the general maps are contracted by the compiler
+    for each kernel). A beam that is partly lost, and one on and near the zero orbit."""
+    E, L = bmx.elements, bmx.lattices
+    p0c, et = L.reference()
+    mk = lambda key, **kw: E.make_element(key, p0c, et, **kw, x_limit=0.02, y_limit=0.02)  # noqa: E731
+    rng = np.random.default_rng(5)
+    general = _general(bmx, kind)
+    eles = []
+    for c in range(10):
+        a, b, w = rng.uniform(0.5, 1.0, 3)
+        eles += [general(w), mk(E.DRIFT, l=0.4 * a), mk(E.QUADRUPOLE, l=0.3, k1=0.3 * a), general(a), general(b),
+                 mk(E.SBEND, l=1.0, g=0.02), mk(E.QUADRUPOLE, l=0.3, k1=-0.3 * b), general(b)]
+    arr = E.to_array(eles + [mk(E.DRIFT, l=0.1)])
+    near = P.random_beam(bmx, 200, 2, scale=1e-3)
+    for k in P.COORDS:
+        near[k][:20] = 0
+    near["pz"][:100] = 0
+    near["beta"] = L.init_beta(near["pz"], p0c, et)
+    for beam in (P.random_beam(bmx, 500, 2, scale=10.0, pz_sigma=5e-4), near):
+        print(f"general cells {kind}", flush=True)
+        want = _track(bmx, ctx, arr, beam, False)
+        got = _track(bmx, ctx, arr, beam, True)
+        assert P.loss_mismatch(got, want).size == 0
+        alive = want["state"] == 1
+        assert alive.sum() > 10
+        assert P.rel_err(got, want, alive) <= 1e-12 * 2 * len(arr)
+
+
+def test_cells_whose_elements_are_of_different_kinds_of_operation(bmx, ctx):
+    """A cell position that is on the short series of the quadrupole in some cells and on the long one
+    in others: the same bits as the generic kernel, which takes each element by its own."""
+    E = bmx.elements
+    p0c, et = bmx.lattices.reference()
+    mk = lambda key, **kw: E.make_element(key, p0c, et, **kw, x_limit=0.02, y_limit=0.02)  # noqa: E731
+    k1 = [0.6, -0.62, 0.61, -0.6] * 3
+    eles = [e for c, k in enumerate(k1) for e in
+            (mk(E.DRIFT, l=0.4), mk(E.QUADRUPOLE, l=0.3, k1=k), mk(E.DRIFT, l=0.2 + 0.01 * c))]
+    print("cells of different operations", flush=True)
+    arr = E.to_array(eles)
+    beam = P.random_beam(bmx, 500, 2, scale=10.0)
+    _same(_track(bmx, ctx, arr, beam, True), _track(bmx, ctx, arr, beam, False))
