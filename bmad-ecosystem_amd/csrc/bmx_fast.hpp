@@ -67,8 +67,11 @@ __device__ __forceinline__ void fast_put_energy(Particle &p, const FastE &en)
 typedef double OpVec __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ OpVec load_op(CP r) { return *(const OpVec BMX_CONST *)r; }
 
-// Bound of (px^2 + py^2)/(1+pz)^2 (angles below 15.6 mrad) in drifts and at both faces of bends.
-constexpr double kFastU2 = 0x1p-12;
+// Bound of u = (px^2 + py^2)/(1+pz)^2 (angles below 44 mrad) in drifts and at both faces of bends:
+// beyond the general maps' own series (31 mrad), so that a beam of large angles is not sent through a
+// run and then element by element for lanes that those take by series. At 15.6 mrad, two terms fewer in
+// the bend, 700 elements at angles of 8 mrad rms took 2.0 to 3.2 times as long as the general maps.
+constexpr double kFastU2 = 0x1p-9;
 // Bound of t = (k1 L^2/(1+pz))^2 of the short quadrupole series.
 constexpr double kFastT = 0x1p-8;
 
@@ -94,7 +97,7 @@ __device__ __forceinline__ void fast_unstable(const FastP &f, const FastE &en, L
 }
 
 // track_a_drift.f90:25-116 by the series of 1/ps - 1 (drift_series with the terms that
-// kFastU2 leaves: the first omitted one, 231/512 u^5 of the sum, is below 4e-19).
+// kFastU2 leaves: the first omitted one, 231/1024 u^6 of q, is below 1.3e-17, 2e-19 at 31 mrad).
 __device__ __forceinline__ void fast_drift(FastP &f, const FastE &en, double L,
                                            LaneMask &bad)
 {
@@ -186,7 +189,7 @@ __device__ __forceinline__ void fast_sextupole(FastP &f, const FastE &en, double
 // (px^2 + py^2)/(1+pz)^2, the orbit turns by theta + (phi_t - phi_f) with
 //   sin(phi_t - phi_f) = (px_t c_f - px_f c_t)/((1+pz) (1 - w)),   w = (py/(1+pz))^2
 // (ux^2 + c^2 = 1 - w at both faces), whose reciprocal is a short series and whose arcsine,
-// below 1/32, another (both to 2e-17): no division. The path length is h (theta + phi_t - phi_f)
+// below 0.089, another (to 3e-17, and 2e-17 of the angle where w is large): no division. The path length is h (theta + phi_t - phi_f)
 // with h = (1+pz)/g, and against the clock's beta L/beta0 it leaves z only L (bq - pz) - h (phi_t
 // - phi_f), without the difference of two terms of the size of L.
 // near: some lane has |pz| < 1e-9; those that are all within 1e-9 of the zero orbit take the
@@ -227,14 +230,16 @@ __device__ __forceinline__ void fast_bend(FastP &f, const FastE &en, const V &r,
     n = n * sf;
     const double br = fma(px, sa, fma(v, omc, en.rel_p * (n - m)));
     f.x = fma(br, inv_g, x * ca);
-    // 1/(1 - w), w < 2^-12
+    // 1/(1 - w): the first omitted term, w^6, is below 6e-17, and only where s is near zero
     double iv = 1.0 + w;
+    iv = fma(w, iv, 1.0);
     iv = fma(w, iv, 1.0);
     iv = fma(w, iv, 1.0);
     iv = fma(w, iv, 1.0);
     const double s = fma(px, 1.0 + n, -(pf * (1.0 + m))) * (iv * en.inv_rp);
     const double s2 = s * s;
-    double q = fma(s2, 0.022372159090909092, 0.030381944444444444);  // 63/2816, 35/1152
+    double q = fma(s2, 0.017352764423076924, 0.022372159090909092);   // 231/13312, 63/2816
+    q = fma(q, s2, 0.030381944444444444);                              // 35/1152
     q = fma(q, s2, 0.044642857142857144);                              // 5/112
     q = fma(q, s2, 0.075);                                              // 3/40
     q = fma(q, s2, 0.16666666666666666);                               // 1/6
