@@ -202,10 +202,10 @@ __device__ __forceinline__ void store_changed(double v, double was, double *__re
 // One element, whole bunch: track1 (track1.f90:44-343) per live particle. Q: the kernel carries
 // the stepped quadrupole and the general bend (built for lattices that hold one).
 //
-// Bound by memory: the state and seven coordinates come in with one wait (a dead particle's
-// coordinates are read as well: waiting for its state first would double the latency), and only
-// what the element changed goes out (a drift 3 of the 7 arrays, a magnet 5). Nine elements of 1e6
-// particles: 336 -> 317 us; registers for 6 waves per SIMD instead of 4 spill, and took 376 us.
+// Bound by memory: only what the element changed goes out (a drift 3 of the 7 arrays, a magnet 5).
+// Nine elements of 1e6 particles: 332 -> 319 us. Reading the coordinates along with the state takes 1%
+// less (315 us), but a beam of dead particles then 1.4 times as long (1e6, nine tenths dead at its
+// end: 90 -> 129 us, now 88). Registers for 6 waves per SIMD instead of 4 spill, and took 376 us.
 template <bool F, int Q>
 __device__ __forceinline__ void track_element_pass(const LatDesc &L, int32_t ie, int32_t turn,
                                                    const BeamPtrs &b, int64_t n,
@@ -213,15 +213,11 @@ __device__ __forceinline__ void track_element_pass(const LatDesc &L, int32_t ie,
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     StepAhead s = F ? step_at(L, ie) : StepAhead{};
-    Particle p;
-    int32_t state = 0;
-    if (i < n) {
-        state = b.state[i];
-        load_particle(p, b, i);
-    }
-    const bool active = state == ST_ALIVE;
+    const bool active = i < n && b.state[i] == ST_ALIVE;
     const LaneMask live = lanes(active);
     if (active) {
+        Particle p;
+        load_particle(p, b, i);
         const Particle was = p;
         refresh_energy(p, L.sp);
         if (!orbit_too_large(p)) {
@@ -247,7 +243,8 @@ __device__ __forceinline__ void track_element_pass(const LatDesc &L, int32_t ie,
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = (uint32_t)__popcll(live);
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned long long t = 0;        for (int w = 0; w < kBlock / 64; w++) t += part[w];
+        unsigned long long t = 0;
+        for (int w = 0; w < kBlock / 64; w++) t += part[w];
         if (t) atomicAdd(work + blockIdx.x % kWorkSlots, t);
     }
 }
