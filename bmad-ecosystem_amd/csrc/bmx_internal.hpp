@@ -143,13 +143,13 @@ struct RunConfig {
 hipError_t enqueue_run(hipStream_t s, RunBuffers &rb, const Group *h_groups, int32_t n_groups,
                        bool upload, int32_t max_turns, const RunConfig &cfg,
                        unsigned long long *d_work);
+// The rounds of the 4-wave cell kernel's resident waves above which a beam runs the 5-wave build.
+constexpr double kPhaseRounds = 1.45;
 // Default waves per SIMD of the tracking kernel: the variant measured fastest on the 901-element
 // ring for each kernel (cell-specialised 4: at most 128 VGPRs, so 4 waves per SIMD are resident,
 // without spilling; generic fast maps 5; reference maps 3, whose 4- and 5-wave builds spill).
 // Cell kernels that carry the stepped quadrupole or the general bend are all built for 2 waves per
 // SIMD (their longer maps would spill otherwise), whichever variant is asked for.
-// The rounds of the 4-wave cell kernel's resident waves above which a beam runs the 5-wave build.
-constexpr double kPhaseRounds = 1.45;
 inline int32_t default_waves(bool fast, const JitKernels *jit = nullptr)
 {
     return jit ? (jit_rare_q(jit) ? 3 : 4) : (fast ? 5 : 3);

@@ -53,7 +53,7 @@ class Context:
     def set_run(self, chunk_turns: int = 5, grid: int = 0, waves: int = 0) -> None:
         """Turns per chunk of bmx_track_turns (0 = one chunk), persistent grid size (0 = device
         occupancy limit) and waves per SIMD of the kernel variant (3, 4 or 5; 0 = chosen per
-        call: on a specialised lattice 5 or 4 by the live particles' count, else 5 with the fast
+        call: on a specialised lattice 5 or 4 by the beam's size, else 5 with the fast
         maps, 3 with the reference maps)."""
         native.call("bmx_ctx_set_run", self.h, int(chunk_turns), int(grid), int(waves))
 

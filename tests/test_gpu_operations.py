@@ -124,7 +124,7 @@ def test_single_elements(bmx, oracle, ctx, ap):
 
 
 def _mixed_ring(bmx, cells=4):
-    """A line of repeated cells of every kind of operation."""
+    """A line of repeated cells of every kind of operation, each element of strengths of its own."""
     e = _elements(bmx, x_limit=0.02, y_limit=0.02, aperture_type=bmx.elements.APERTURE_ELLIPTICAL)
     cell = [e["drift"], e["quad_weak"], e["sext_1"], e["marker"], e["kicker_thick"], e["bend"], e["quad_mid"],
             e["quad_corrector"], e["sext_3"], e["bend_k1"], e["drift"], e["kicker_thin"], e["sext_offset"],
@@ -136,6 +136,9 @@ def _mixed_ring(bmx, cells=4):
     arr["k2"] *= 0.3
     arr["hkick"] *= 0.1
     arr["vkick"] *= 0.1
+    rng = np.random.default_rng(31)
+    for f in ("k1", "k2", "g", "hkick", "vkick", "x_offset", "y_offset"):
+        arr[f] *= 1 + 0.1 * rng.uniform(-1, 1, len(arr))
     return arr
 
 
