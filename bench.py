@@ -282,6 +282,8 @@ def main():
                             "default run, " + traffic_file(special),
             "traffic_algorithmic": bytes_alg,
             "flop_per_particle_element": flops,
+            "flop_note": "operations of the reference's formulas; the kernel executes fewer: "
+                         "profiles/bmx_cell_tiles_ring1_1e6_valu.md",
             "kernel": " then ".join(kernels), "kernel_steps": kernels,
             "kernel_ms_avg": kernel_ms / max(launches, 1),
             "launches": launches, "step_ms": [float(x) for x in launch_ms],
