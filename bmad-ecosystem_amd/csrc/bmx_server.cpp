@@ -36,6 +36,7 @@ constexpr int64_t kBytesPerParticle = 7 * 8 + 3 * 4 + 2 * (int64_t)kPackedBytes;
 struct Request {
     int64_t id = 0;
     const bmx_lattice *lat = nullptr;
+    RadCfg rad{};  // the lattice's radiation settings when the request was submitted
     int64_t n = 0;
     int32_t n_turns = 0, turn0 = 0, done_turns = 0, chunks = 0;
     bmx_beam_view in{}, out{};
@@ -262,6 +263,7 @@ void bmx_server::run()
                 const bmx_lattice::View v = r->lat->view();
                 j = i == 0 || v.jit == j ? v.jit : nullptr;
                 g.lat = v.desc;
+                g.lat.sp.rad = r->rad;
                 g.b = at(r->off);
                 g.n = (uint32_t)r->n;
                 g.list_off = (uint32_t)r->off;
@@ -414,6 +416,7 @@ int32_t bmx_server_submit(bmx_server *S, const bmx_lattice *lat, const bmx_beam_
     Request *r = new (std::nothrow) Request();
     if (!r) return set_error(BMX_ERR_NOMEM, "bmx_server_submit: host allocation");
     r->lat = lat;
+    r->rad = lat->view().desc.sp.rad;
     r->n = n;
     r->n_turns = n_turns;
     r->turn0 = turn0;

@@ -225,7 +225,8 @@ int32_t bmx_lattice_validate(const bmx_ele *eles, int32_t n_ele, double mc2, int
  * variants) share one compiled kernel. Used by the fast-map runs of bmx_track_turns and
  * bmx_batch_track; the maps are the generic kernel's, so results agree with it to rounding
  * (losses identical in the parity tests). BMX_ERR_UNSUPPORTED when no
- * such cell exists (the generic kernel is then used). No counterpart in the reference, whose
+ * such cell exists (the generic kernel is then used). A server may be tracking through the
+ * lattice meanwhile: its next chunk takes the new kernels up. No counterpart in the reference, whose
  * element loop is track_all (bmad/code/track_all.f90:1) over the generic element dispatch. */
 int32_t bmx_lattice_specialize(bmx_lattice *lat);
 /* Number of elements and bit set of element kinds present (bit = key). */

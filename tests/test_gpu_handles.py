@@ -58,7 +58,7 @@ def test_plain_turns_of_replaced_lattices(bmx, ctx):
     off = mk(E.QUADRUPOLE, l=0.3, k1=-0.2, x_offset=1e-4, tilt=0.1)
     beam = P.random_beam(bmx, 300, 6, scale=10.0, pz_sigma=1e-3)
     gb = T.Beam.from_host(ctx, beam)
-    for round_ in range(2):
+    for again in range(2):
         for name, cell, rad in (("plain", [d, q, d, b], False), ("stepped", [d, q2, d, b], False),
                                 ("radiating", [d, q, d, b], True), ("offset", [d, off, d, b], False),
                                 ("stepped radiating", [d, q2, d, b], True), ("drifts", [d] * 4, False)):
@@ -71,7 +71,7 @@ def test_plain_turns_of_replaced_lattices(bmx, ctx):
             for seed in ((3, 4) if rad else (0,)):
                 if seed == 4:
                     lat.set_radiation(T.rad_config(True, True, seed=seed))
-                print(f"plain turns {name} round {round_} seed {seed}", flush=True)
+                print(f"plain turns {name} pass {again} seed {seed}", flush=True)
                 outs = []
                 for track in (T.track_beam_plain, T.track_beam):
                     gb.upload(beam)
@@ -84,3 +84,28 @@ def test_plain_turns_of_replaced_lattices(bmx, ctx):
                 assert P.rel_err(outs[0], outs[1], alive) <= 1e-12 * 2 * len(arr), name
             lat.close()
     gb.close()
+
+
+def test_served_requests_keep_their_radiation_settings(bmx, ctx):
+    """A lattice's radiation settings changed while a request through it waits or runs (chunks of 2
+    turns): the request keeps those it was submitted with, the next one has the new ones; each
+    bit-identical to its beam alone with them."""
+    E, T = bmx.elements, bmx.tracking
+    arr = E.to_array(bmx.lattices.ring1(n_cells=6))
+    maps = T.rad_maps(len(arr))
+    bends = np.nonzero(arr["key"] == E.SBEND)[0]
+    maps["damp_dmat"][bends, :, 5, 5] = -1e-4
+    maps["stoc_mat"][bends, :, 5, 5] = 1e-5
+    cfgs = [T.rad_config(True, True, seed=1), T.rad_config(True, True, scale=2.0, seed=2)]
+    beam = P.random_beam(bmx, 400, 3)
+    lat = T.Lattice(ctx, arr, rad_maps=maps, rad=cfgs[0])
+    server = T.Server(ctx, 64 << 20, chunk_turns=2)
+    print("served radiation settings", flush=True)
+    first = server.submit(lat, beam, 60)
+    lat.set_radiation(cfgs[1])
+    second = server.submit(lat, beam, 60)
+    outs = [server.wait(r)[0] for r in (first, second)]
+    server.close()
+    lat.close()
+    for out, cfg in zip(outs, cfgs):
+        _same(out, T.track_beam_host(arr, beam, 60, rad_maps=maps, rad=cfg))
